@@ -298,6 +298,26 @@ int linatt_kata_gen_update(const void* k, const void* v, const float* c, float* 
                            int init, int B, int T, int H, int dk, int dv, int num_groups,
                            int variant, float scale, int dtype, void* stream);
 
+/* linatt_kata_gen_readout / linatt_kata_gen_update with the work of a small
+ * batch split over more workgroups: the readout's state rows, the update's
+ * tokens, each split's partial sums (float32) in the workspace and added in
+ * split order by a second launch.  workspace: 16-byte aligned, at least
+ * linatt_kata_gen_{readout,update}_workspace_bytes bytes, 0 where no split
+ * pays or applies (float32 inputs, large batches; it may then be NULL).  Same
+ * results as the unsplit calls up to the float32 summation order. */
+size_t linatt_kata_gen_readout_workspace_bytes(int B, int T, int H, int dk, int num_groups,
+                                               int variant, int dtype);
+int linatt_kata_gen_readout_split(const void* q, const float* c, const float* S, const float* z,
+                                  void* o, float* den, void* workspace, size_t workspace_bytes,
+                                  int B, int T, int H, int dk, int dv, int num_groups, int variant,
+                                  float scale, float eps, int dtype, void* stream);
+size_t linatt_kata_gen_update_workspace_bytes(int B, int T, int H, int dk, int num_groups,
+                                              int variant, int dtype);
+int linatt_kata_gen_update_split(const void* k, const void* v, const float* c, float* S, float* z,
+                                 int init, void* workspace, size_t workspace_bytes, int B, int T,
+                                 int H, int dk, int dv, int num_groups, int variant, float scale,
+                                 int dtype, void* stream);
+
 /* 1 if the state-form kernels are compiled for the combination, else 0. */
 int linatt_kata_state_supported(int dtype, int dk, int dv, int num_groups);
 

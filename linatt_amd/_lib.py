@@ -67,6 +67,10 @@ SIGNATURES = {
     "linatt_kata_gen_decode_split": (_i, [_vp] * 8 + [_sz] + [_i] * 6 + [_f, _f, _i, _vp]),
     "linatt_kata_gen_readout": (_i, [_vp] * 6 + [_i] * 7 + [_f, _f, _i, _vp]),
     "linatt_kata_gen_update": (_i, [_vp] * 5 + [_i] * 8 + [_f, _i, _vp]),
+    "linatt_kata_gen_readout_workspace_bytes": (_sz, [_i] * 7),
+    "linatt_kata_gen_readout_split": (_i, [_vp] * 7 + [_sz] + [_i] * 7 + [_f, _f, _i, _vp]),
+    "linatt_kata_gen_update_workspace_bytes": (_sz, [_i] * 7),
+    "linatt_kata_gen_update_split": (_i, [_vp] * 5 + [_i, _vp, _sz] + [_i] * 7 + [_f, _i, _vp]),
     "linatt_kata_prefill_workspace_bytes": (_sz, [_i] * 8),
     "linatt_kata_prefill": (_i, [_vp] * 8 + [_i] * 6 + [_f, _f, _i, _i, _i, _vp]),
     "linatt_kata_prefill_state": (_i, [_vp] * 10 + [_i] * 6 + [_f, _f, _i, _i, _i, _vp]),

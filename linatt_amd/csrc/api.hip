@@ -1195,36 +1195,110 @@ int linatt_kata_gen_decode_split(const void* q, const void* k, const void* v, co
   return gen_state_launch(fn, a, KATA_GEN_DECODE, dtype, stream);
 }
 
-int linatt_kata_gen_readout(const void* q, const float* c, const float* S, const float* z,
-                            void* o, float* den, int B, int T, int H, int dk, int dv,
-                            int num_groups, int variant, float scale, float eps, int dtype,
-                            void* stream) {
+// the workspace of a split call: its size and alignment, then a.part
+static int gen_state_split_ws(const char* fn, const char* query, KataGenStateArgs& a, size_t need, void* ws, size_t ws_bytes) {
+  if (!need) return LINATT_OK;
+  if (!ws || ws_bytes < need) return fail(LINATT_EINVAL, std::string(fn) + ": workspace smaller than " + query);
+  if (!aligned16(ws)) return fail(LINATT_EINVAL, std::string(fn) + ": workspace must be 16-byte aligned");
+  a.part = reinterpret_cast<float*>(ws);
+  return LINATT_OK;
+}
+static bool half_dtype(int dtype) { return dtype == LINATT_BFLOAT16 || dtype == LINATT_FLOAT16; }
+
+static int gen_readout_splits(const KataGenStateArgs& a, int dtype) {
+  if (!half_dtype(dtype)) return 1;
+  return kata_gen_readout_splits((int64_t)a.B * a.H, a.T, a.E, a.M, a.sum, a.tri);
+}
+static int gen_update_splits(const KataGenStateArgs& a, int dtype) {
+  return half_dtype(dtype) ? kata_gen_update_splits((int64_t)a.B * a.H, a.sum ? 1 : a.M, a.E, a.T) : 1;
+}
+static size_t gen_readout_ws(const KataGenStateArgs& a, int ns) {
+  return ns > 1 ? (size_t)ns * a.B * a.T * a.H * kGenDecPart * sizeof(float) : 0;
+}
+static size_t gen_update_ws(const KataGenStateArgs& a, int ns) {
+  return ns > 1 ? (size_t)ns * a.B * a.H * a.P * 65 * sizeof(float) : 0;
+}
+
+static int gen_readout_impl(const char* fn, const void* q, const float* c, const float* S, const float* z,
+                            void* o, float* den, int B, int T, int H, int dk, int dv, int num_groups,
+                            int variant, float scale, float eps, int dtype, void* stream, bool split,
+                            void* ws, size_t ws_bytes) {
   g_last_error.clear();
-  const char* fn = "linatt_kata_gen_readout";
   KataGenStateArgs a{};
   int st = gen_state_args(fn, a, B, T, H, dk, dv, num_groups, variant, scale, eps, dtype);
   if (st) return st;
   if (!q || !S || !z || !o || !den) return fail(LINATT_EINVAL, std::string(fn) + ": null tensor pointer");
   if (!aligned16(q) || !aligned16(S) || !aligned16(o))
     return fail(LINATT_EINVAL, std::string(fn) + ": q, S and o must be 16-byte aligned");
+  if (split) {
+    a.nsplit = gen_readout_splits(a, dtype);
+    st = gen_state_split_ws(fn, "linatt_kata_gen_readout_workspace_bytes", a, gen_readout_ws(a, a.nsplit), ws, ws_bytes);
+    if (st) return st;
+  }
   a.q = q; a.c = c; a.S = const_cast<float*>(S); a.z = const_cast<float*>(z); a.o = o; a.den = den;
   return gen_state_launch(fn, a, KATA_GEN_READOUT, dtype, stream);
 }
 
-int linatt_kata_gen_update(const void* k, const void* v, const float* c, float* S, float* z,
-                           int init, int B, int T, int H, int dk, int dv, int num_groups,
-                           int variant, float scale, int dtype, void* stream) {
+int linatt_kata_gen_readout(const void* q, const float* c, const float* S, const float* z,
+                            void* o, float* den, int B, int T, int H, int dk, int dv,
+                            int num_groups, int variant, float scale, float eps, int dtype,
+                            void* stream) {
+  return gen_readout_impl("linatt_kata_gen_readout", q, c, S, z, o, den, B, T, H, dk, dv, num_groups, variant,
+                          scale, eps, dtype, stream, false, nullptr, 0);
+}
+
+size_t linatt_kata_gen_readout_workspace_bytes(int B, int T, int H, int dk, int num_groups, int variant, int dtype) {
+  KataGenStateArgs a{};
+  if (gen_state_args("", a, B, T, H, dk, 64, num_groups, variant, 1.f, 1.f, dtype)) return 0;
+  return gen_readout_ws(a, gen_readout_splits(a, dtype));
+}
+
+int linatt_kata_gen_readout_split(const void* q, const float* c, const float* S, const float* z,
+                                  void* o, float* den, void* workspace, size_t workspace_bytes, int B,
+                                  int T, int H, int dk, int dv, int num_groups, int variant, float scale,
+                                  float eps, int dtype, void* stream) {
+  return gen_readout_impl("linatt_kata_gen_readout_split", q, c, S, z, o, den, B, T, H, dk, dv, num_groups, variant,
+                          scale, eps, dtype, stream, true, workspace, workspace_bytes);
+}
+
+static int gen_update_impl(const char* fn, const void* k, const void* v, const float* c, float* S, float* z,
+                           int init, int B, int T, int H, int dk, int dv, int num_groups, int variant,
+                           float scale, int dtype, void* stream, bool split, void* ws, size_t ws_bytes) {
   g_last_error.clear();
-  const char* fn = "linatt_kata_gen_update";
   KataGenStateArgs a{};
   int st = gen_state_args(fn, a, B, T, H, dk, dv, num_groups, variant, scale, 1.f, dtype);
   if (st) return st;
   if (!k || !v || !S || !z) return fail(LINATT_EINVAL, std::string(fn) + ": null tensor pointer");
   if (!aligned16(S) || !aligned16(k) || !aligned16(v))
     return fail(LINATT_EINVAL, std::string(fn) + ": k, v and S must be 16-byte aligned");
+  if (split) {
+    a.nsplit = gen_update_splits(a, dtype);
+    st = gen_state_split_ws(fn, "linatt_kata_gen_update_workspace_bytes", a, gen_update_ws(a, a.nsplit), ws, ws_bytes);
+    if (st) return st;
+  }
   a.k = k; a.v = v; a.c = c; a.S = S; a.z = z; a.init = init ? 1 : 0;
   return gen_state_launch(fn, a, KATA_GEN_UPDATE, dtype, stream);
 }
 
+int linatt_kata_gen_update(const void* k, const void* v, const float* c, float* S, float* z,
+                           int init, int B, int T, int H, int dk, int dv, int num_groups,
+                           int variant, float scale, int dtype, void* stream) {
+  return gen_update_impl("linatt_kata_gen_update", k, v, c, S, z, init, B, T, H, dk, dv, num_groups, variant, scale,
+                         dtype, stream, false, nullptr, 0);
+}
+
+size_t linatt_kata_gen_update_workspace_bytes(int B, int T, int H, int dk, int num_groups, int variant, int dtype) {
+  KataGenStateArgs a{};
+  if (gen_state_args("", a, B, T, H, dk, 64, num_groups, variant, 1.f, 1.f, dtype)) return 0;
+  return gen_update_ws(a, gen_update_splits(a, dtype));
+}
+
+int linatt_kata_gen_update_split(const void* k, const void* v, const float* c, float* S, float* z,
+                                 int init, void* workspace, size_t workspace_bytes, int B, int T, int H,
+                                 int dk, int dv, int num_groups, int variant, float scale, int dtype,
+                                 void* stream) {
+  return gen_update_impl("linatt_kata_gen_update_split", k, v, c, S, z, init, B, T, H, dk, dv, num_groups, variant,
+                         scale, dtype, stream, true, workspace, workspace_bytes);
+}
 
 }  // extern "C"

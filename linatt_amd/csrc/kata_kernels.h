@@ -138,6 +138,55 @@ inline int kata_gen_decode_splits(int BH, int P) {
   return ns < 1 ? 1 : ns;
 }
 
+// Splits of the 16-bit update's tokens and of the 16-bit readout's state rows
+// over workgroups (kata_state_gen.hip).  Unsplit, a workgroup walks every
+// 64-token chunk (every stage of 64 rows) in turn, and a small batch is a few
+// dozen such chains.  A split shortens the chain but writes one more partial
+// sum, read back by a second launch: the count taken is the one with the
+// least of chain + second launch + partial bytes, as measured on one MI355X
+// (a chunk 1.9 us; a stage 1.5 us, 0.5 us more per further group of the sum
+// score; the second launch 4 us; the partials at 4.5 TB/s both ways), at most
+// 768 workgroups in all (three per CU, 44-47 KB of LDS each).  B1 H12, us,
+// unsplit -> split: update at T = 1500 concat M = 1 47 -> 32, sum M = 4
+// 47 -> 16; readout at T = 200 concat M = 1 62 -> 19; left unsplit, since
+// split it is slower: update at T = 200 concat M = 1 (12 against 17).
+constexpr int kGenMaxSplit = 16;
+inline int kata_gen_best_split(int64_t wgs, int steps, double step_us, double part_bytes) {
+  int best = 1;
+  double t_best = steps * step_us;
+  for (int ns = 2; ns <= kGenMaxSplit && ns <= steps && wgs * ns <= 768; ++ns) {
+    const int per = (steps + ns - 1) / ns;
+    if ((steps + per - 1) / per != ns) continue;  // a split would be empty
+    const double t = per * step_us + 4. + ns * part_bytes * (2. / 4.5e6);
+    if (t < t_best) {
+      t_best = t;
+      best = ns;
+    }
+  }
+  return best;
+}
+// row tiles x column halves of the update's grid per (b, h): 256 rows and
+// both column halves per workgroup; a state of at most 256 rows that would
+// leave CUs idle takes 128 rows and one half (more workgroups, each streaming
+// every token: the staging, not the products, is this kernel's cost, so larger
+// states keep the 256-row tiles)
+inline bool kata_gen_update_small(int64_t BH, int P) {
+  return !(P > 256 || BH * ((P + 255) / 256) >= 512);
+}
+// from the score's packed row count, whatever the state's layout, so that the
+// packed rows equal the full layout's bit for bit (the same sums in the same
+// order)
+inline int kata_gen_update_splits(int64_t BH, int groups, int E, int T) {
+  const int P = groups * (E * (E + 1) / 2);
+  const int64_t wgs = BH * (kata_gen_update_small(BH, P) ? 2 * ((P + 127) / 128) : (P + 255) / 256);
+  return kata_gen_best_split(wgs, (T + 63) / 64, 1.9, BH * (P * 260.));
+}
+inline int kata_gen_readout_splits(int64_t BH, int T, int E, int M, int sum, int tri) {
+  // stages of four 16-row chunks (readout_chunk)
+  const int stages = (sum ? 1 : M) * (tri ? E * (E + 16) / 32 : E * (E / 16)) / 4;
+  return kata_gen_best_split(BH * ((T + 127) / 128), stages, 1.5 + (sum ? 0.5 * (M - 1) : 0.), BH * (T * 272.));
+}
+
 struct KataDecodeArgs {
   const void* q;   // (B, H, DK)
   const void* k;
@@ -169,8 +218,11 @@ struct KataGenStateArgs {
   int B, T, H, dk, E, lgE, M, P, sum;
   int tri;           // 1: packed rows, one per unordered pair a <= b of each group
   int TE;            // packed rows per group, E (E + 1) / 2
-  int nsplit;        // decode: workgroups per (b, h) (1: o written directly)
-  float* part;       // decode, nsplit > 1: (B*H, nsplit, kGenDecPart) partial num (64) and den
+  int nsplit;        // decode: workgroups per (b, h); update: token splits; readout: row splits (1: direct)
+  // nsplit > 1, float32 partials.  decode: (B*H, nsplit, kGenDecPart), num (64)
+  // and den; readout: (nsplit, B, T, H, kGenDecPart) likewise; update:
+  // (nsplit, B*H, P, 64) of S, then (nsplit, B*H, P) of z
+  float* part;
   float scale, eps;
   int init;          // update: 1 = add to f_T S, 0 = start from zero
 };

@@ -422,7 +422,11 @@ __global__ __launch_bounds__(256) void kata_gen_update_mfma_kernel(KataGenStateA
   __shared__ __attribute__((aligned(16))) __bf16 Vt[32 * NCB][kUpVp];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, hh = lane >> 5, cl = lane & 31;
   const int bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
-  const int n0c = NCB == 2 ? 0 : 32 * blockIdx.z;  // first state column of this workgroup
+  // grid z: the token split, with NCB = 1 also the column half
+  const int sp_i = NCB == 2 ? blockIdx.z : blockIdx.z >> 1;
+  const int n0c = NCB == 2 ? 0 : 32 * (blockIdx.z & 1);  // first state column of this workgroup
+  const int per = (((a.T + kUpTok - 1) / kUpTok + a.nsplit - 1) / a.nsplit) * kUpTok;  // tokens per split
+  const int s_lo = sp_i * per, s_hi = min(a.T, s_lo + per);
   const int pw = blockIdx.y * 128 * RB + 32 * RB * w;  // this wave's first row
   const bool wlive = pw < a.P;
   int ia[RB], ib[RB];
@@ -544,15 +548,39 @@ __global__ __launch_bounds__(256) void kata_gen_update_mfma_kernel(KataGenStateA
       }
     }
   };
-  load(pf, 0);
-  for (int s0 = 0; s0 < a.T; s0 += kUpTok) {
+  load(pf, s_lo);
+  for (int s0 = s_lo; s0 < s_hi; s0 += kUpTok) {
     __syncthreads();  // the previous tokens are consumed
     stage(pf, s0);
     __syncthreads();
-    if (s0 + kUpTok < a.T) load(pf, s0 + kUpTok);
+    if (s0 + kUpTok < s_hi) load(pf, s0 + kUpTok);
     compute();
   }
   if (!wlive) return;
+  if (a.nsplit > 1) {
+    // this split's partial sums; kata_gen_update_finish_kernel adds them
+    const size_t BH = gridDim.x;
+    float* Sp = a.part + ((size_t)sp_i * BH + bh) * a.P * kGenDV;
+    float* zp = a.part + (size_t)a.nsplit * BH * a.P * kGenDV + ((size_t)sp_i * BH + bh) * a.P;
+#pragma unroll
+    for (int k = 0; k < RB; ++k) {
+      zacc[k] += __shfl_xor(zacc[k], 32);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int p = pw + 32 * k + 8 * i + 4 * hh + r;
+          if (p < a.P) {
+#pragma unroll
+            for (int cb = 0; cb < NCB; ++cb)
+              Sp[(size_t)p * kGenDV + n0c + 32 * cb + cl] = acc[k][cb][4 * i + r];
+          }
+        }
+      const int p = pw + 32 * k + cl;
+      if (hh == 0 && live[k] && n0c == 0) zp[p] = zacc[k];
+    }
+    return;
+  }
   const float fT = a.c ? __expf(cT) : 1.f;
   float* S = a.S + (size_t)bh * a.P * kGenDV;
   float* z = a.z + (size_t)bh * a.P;
@@ -577,6 +605,35 @@ __global__ __launch_bounds__(256) void kata_gen_update_mfma_kernel(KataGenStateA
     const int p = pw + 32 * k + cl;
     if (hh == 0 && live[k] && n0c == 0) z[p] = (a.init ? fT * z[p] : 0.f) + zacc[k];
   }
+}
+
+// The split update's state: per state row (16 threads, four columns each) the
+// splits' partial sums added in split order,
+//   S <- (init ? f_T S : 0) + sum_i part_i,  z likewise.
+__global__ __launch_bounds__(256) void kata_gen_update_finish_kernel(KataGenStateArgs a) {
+  const size_t BH = (size_t)a.B * a.H, rows = BH * a.P;
+  const size_t row = (size_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int c4 = threadIdx.x & 15;
+  if (row >= rows) return;
+  const int bh = (int)(row / a.P), b = bh / a.H, h = bh % a.H;
+  const float fT = a.init ? (a.c ? __expf(a.c[((int64_t)b * a.T + a.T - 1) * a.H + h]) : 1.f) : 0.f;
+  const float* pz = a.part + (size_t)a.nsplit * rows * kGenDV;
+  float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+  float zz = 0.f;
+#pragma unroll 4
+  for (int i = 0; i < a.nsplit; ++i) {
+    const float4 y = *reinterpret_cast<const float4*>(a.part + (i * rows + row) * kGenDV + 4 * c4);
+    x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w;
+    if (c4 == 0) zz += pz[i * rows + row];
+  }
+  float4* sp = reinterpret_cast<float4*>(a.S + row * kGenDV + 4 * c4);
+  if (a.init) {
+    const float4 o = *sp;
+    x.x += fT * o.x; x.y += fT * o.y; x.z += fT * o.z; x.w += fT * o.w;
+    if (c4 == 0) zz += fT * a.z[row];
+  }
+  *sp = x;
+  if (c4 == 0) a.z[row] = zz;
 }
 
 // Continued prefill's state part for 16-bit inputs, by MFMA: per (b, h, 128
@@ -663,6 +720,9 @@ __global__ __launch_bounds__(256) void kata_gen_readout_mfma_kernel(KataGenState
   const int nb = a.E >> 4;
   const int cpg = a.tri ? a.E * (a.E + 16) / 32 : a.E * nb;  // chunks per group
   const int nch = (a.sum ? 1 : a.M) * cpg;
+  // this workgroup's chunks (blockIdx.z: the row split), whole stages of four
+  const int cper = ((nch / 4 + a.nsplit - 1) / a.nsplit) * 4;
+  const int c_lo = blockIdx.z * cper, c_hi = min(nch, c_lo + cper);
   for (int c = tid; c < cpg; c += 256) Ctab[c] = readout_chunk(a, c);
   __syncthreads();
   // thread (rp, cg) = (tid % 32, tid / 32): rows 2 rp, 2 rp + 1 of the four
@@ -735,12 +795,12 @@ __global__ __launch_bounds__(256) void kata_gen_readout_mfma_kernel(KataGenState
   const QT* qrow = Qs + (32 * w + cl) * kRoQp;
   f32x16 acc0{}, acc1{};
   float dacc = 0.f;
-  load(0);
-  for (int c0 = 0; c0 < nch; c0 += kRoRows / 16) {
+  load(c_lo);
+  for (int c0 = c_lo; c0 < c_hi; c0 += kRoRows / 16) {
     __syncthreads();  // the previous rows are consumed (and Qs is complete)
     stage();
     __syncthreads();
-    if (c0 + kRoRows / 16 < nch) load(c0 + kRoRows / 16);
+    if (c0 + kRoRows / 16 < c_hi) load(c0 + kRoRows / 16);
 #pragma unroll
     for (int kk = 0; kk < kRoRows / 16; ++kk) {
       const int2 ci = Ci[kk];
@@ -774,6 +834,24 @@ __global__ __launch_bounds__(256) void kata_gen_readout_mfma_kernel(KataGenState
   // den part of query 32 w + l % 32: the two lane halves; then every lane
   // reads the queries of its C-layout rows
   dacc += __shfl_xor(dacc, 32);
+  if (a.nsplit > 1) {
+    // this split's partial numerators and denominators; kata_gen_readout_finish_kernel adds them
+    const size_t nrow = (size_t)a.B * a.T * a.H;
+    float* pt = a.part + blockIdx.z * nrow * kGenDecPart;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = t0 + 32 * w + 8 * i + 4 * hh + r;
+        if (t >= a.T) continue;
+        float* row = pt + (((size_t)b * a.T + t) * a.H + h) * kGenDecPart;
+        row[cl] = acc0[4 * i + r];
+        row[32 + cl] = acc1[4 * i + r];
+      }
+    const int t = t0 + 32 * w + cl;
+    if (hh == 0 && t < a.T) pt[(((size_t)b * a.T + t) * a.H + h) * kGenDecPart + kGenDV] = dacc;
+    return;
+  }
   // the 16-bit tile holds q, not q~: the scale multiplies the sums
   const float fs = kQ16 ? a.scale : 1.f;
   if (hh == 0) Dq[w][cl] = dacc;
@@ -805,6 +883,31 @@ __global__ __launch_bounds__(256) void kata_gen_readout_mfma_kernel(KataGenState
   }
 }
 
+// The split readout's combination with the flash forward's (o, den): one wave
+// per (b, t, h) row, a lane per column, the partials added in split order.
+// fs: the scale that the partial sums lack (the 16-bit query tile).
+template <typename T>
+__global__ __launch_bounds__(256) void kata_gen_readout_finish_kernel(KataGenStateArgs a, float fs) {
+  const size_t nrow = (size_t)a.B * a.T * a.H;
+  const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int n = threadIdx.x & 63;
+  if (row >= nrow) return;
+  const float* pt = a.part + row * kGenDecPart;
+  float num = 0.f, dacc = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < a.nsplit; ++s) {
+    num += pt[s * nrow * kGenDecPart + n];
+    dacc += pt[s * nrow * kGenDecPart + kGenDV];
+  }
+  const float fd = (a.c ? __expf(a.c[row]) : 1.f) * fs;
+  const float df = a.den[row];
+  const float dsc = fmaxf(df + fd * dacc, a.eps);
+  T* orow = (T*)a.o + row * kGenDV;
+  orow[n] = (T)(((float)orow[n] * df + fd * num) / dsc);
+  // every lane of the row's wave has read den
+  if (n == 0) a.den[row] = dsc;
+}
+
 // the sum score's group count as a template argument where it is 2, 4 or 8
 // (so the group loop unrolls), -1 for the other counts dk <= 128 allows
 // (3, 5, 6, 7: a loop bounded at run time); the sum score over one group is
@@ -826,7 +929,7 @@ hipError_t launch_kata_gen_state(const KataGenStateArgs& a, int which, hipStream
     if (a.nsplit > 1) kata_gen_decode_finish_kernel<T><<<dim3(BH), dim3(kGenDV), 0, stream>>>(a);
   } else if (which == KATA_GEN_READOUT) {
     if constexpr (sizeof(T) == 2) {
-      const dim3 grid(BH, (a.T + 127) / 128);
+      const dim3 grid(BH, (a.T + 127) / 128, a.nsplit);
       by_sum_groups(a, [&](auto ms) {
         if (a.dk <= 64)
           kata_gen_readout_mfma_kernel<T, decltype(ms)::value, 64><<<grid, dim3(256), 0, stream>>>(a);
@@ -834,22 +937,23 @@ hipError_t launch_kata_gen_state(const KataGenStateArgs& a, int which, hipStream
           kata_gen_readout_mfma_kernel<T, decltype(ms)::value, 128><<<grid, dim3(256), 0, stream>>>(a);
         return hipSuccess;
       });
+      if (a.nsplit > 1)
+        kata_gen_readout_finish_kernel<T><<<dim3((unsigned)(((int64_t)BH * a.T + 3) / 4)), dim3(256), 0, stream>>>(
+            a, a.dk <= 64 ? 1.f : a.scale);
     } else {
       kata_gen_readout_kernel<T><<<dim3(BH, (a.T + 63) / 64), dim3(256), 0, stream>>>(a);
     }
   } else if constexpr (sizeof(T) == 2) {
-    // 256 rows and both column halves per workgroup; a state of at most
-    // 256 rows that would leave CUs idle takes 128 rows and one half (more
-    // workgroups, each streaming every token: the staging, not the products,
-    // is this kernel's cost, so larger states keep the 256-row tiles)
     by_sum_groups(a, [&](auto ms) {
       constexpr int MS = decltype(ms)::value;
-      if (a.P > 256 || (int64_t)BH * ((a.P + 255) / 256) >= 512)
-        kata_gen_update_mfma_kernel<T, MS, 2, 2><<<dim3(BH, (a.P + 255) / 256), dim3(256), 0, stream>>>(a);
+      if (kata_gen_update_small(BH, a.P))
+        kata_gen_update_mfma_kernel<T, MS, 1, 1><<<dim3(BH, (a.P + 127) / 128, 2 * a.nsplit), dim3(256), 0, stream>>>(a);
       else
-        kata_gen_update_mfma_kernel<T, MS, 1, 1><<<dim3(BH, (a.P + 127) / 128, 2), dim3(256), 0, stream>>>(a);
+        kata_gen_update_mfma_kernel<T, MS, 2, 2><<<dim3(BH, (a.P + 255) / 256, a.nsplit), dim3(256), 0, stream>>>(a);
       return hipSuccess;
     });
+    if (a.nsplit > 1)
+      kata_gen_update_finish_kernel<<<dim3((unsigned)(((int64_t)BH * a.P + 15) / 16)), dim3(256), 0, stream>>>(a);
   } else {
     kata_gen_update_kernel<T><<<dim3(BH, (a.P + 63) / 64), dim3(256), 0, stream>>>(a);
   }

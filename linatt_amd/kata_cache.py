@@ -203,16 +203,24 @@ def _generic(q, k, v, state, M, scale, eps, variant, c, offset):
         return o[:, None], KataState(S, z, offset + 1, variant, M)
     # the call's own tokens by the flash forward, then the stored state's part
     o, den = _kata_fwd(q, k, v, M, sc, variant, cf)
+    # a small batch splits the readout's state rows and the update's tokens
+    # over several workgroups (float32 partial sums in a scratch of the call)
+    def scratch(query):
+        nws = query(B, T, H, dk, M, var, code)
+        return (torch.empty(nws, device=q.device, dtype=torch.uint8) if nws else None), nws
+
     if state is not None:
-        _lib.check("linatt_kata_gen_readout", L.linatt_kata_gen_readout(
+        ws, nws = scratch(L.linatt_kata_gen_readout_workspace_bytes)
+        _lib.check("linatt_kata_gen_readout_split", L.linatt_kata_gen_readout_split(
             _lib.ptr(q), _lib.ptr(cf), _lib.ptr(S), _lib.ptr(z), _lib.ptr(o), _lib.ptr(den),
-            B, T, H, dk, dv, M, var, sc, float(eps), code, sp))
+            _lib.ptr(ws), nws, B, T, H, dk, dv, M, var, sc, float(eps), code, sp))
     else:
         S = torch.empty(B, H, P, dv, device=q.device, dtype=torch.float32)
         z = torch.empty(B, H, P, device=q.device, dtype=torch.float32)
-    _lib.check("linatt_kata_gen_update", L.linatt_kata_gen_update(
+    ws, nws = scratch(L.linatt_kata_gen_update_workspace_bytes)
+    _lib.check("linatt_kata_gen_update_split", L.linatt_kata_gen_update_split(
         _lib.ptr(k), _lib.ptr(v), _lib.ptr(cf), _lib.ptr(S), _lib.ptr(z),
-        1 if state is not None else 0, B, T, H, dk, dv, M, var, sc, code, sp))
+        1 if state is not None else 0, _lib.ptr(ws), nws, B, T, H, dk, dv, M, var, sc, code, sp))
     return o, KataState(S, z, offset + T, variant, M)
 
 

@@ -332,3 +332,70 @@ def test_split_decode_equals_decode(dk, M, variant, packed, decay):
     err = mar(o2, o1)
     print(f"  o split vs one workgroup {err:.1e}", flush=True)
     assert err < 1e-2
+
+
+@pytest.mark.parametrize("dk,M,variant,packed,decay,dtype", [
+    (64, 1, "concat", True, False, torch.bfloat16), (64, 1, "concat", False, False, torch.float16),
+    (64, 2, "sum", True, False, torch.bfloat16), (64, 4, "sum", True, False, torch.bfloat16),
+    (64, 2, "concat", True, True, torch.bfloat16), (128, 2, "concat", True, True, torch.float16),
+    (16, 1, "concat", True, False, torch.bfloat16)])
+@pytest.mark.parametrize("T", [1, 64, 255, 257, 1500])
+def test_split_update_readout_equal_unsplit(dk, M, variant, packed, decay, dtype, T):
+    """``linatt_kata_gen_update_split`` / ``_readout_split`` against the
+    unsplit calls, from a stored state: the same products, summed in another
+    order.  Bounds: two float32 sums of n terms differ by at most
+    2 n 2^-24 sum|terms| (S, z, and with them den); o is rounded once more to
+    the dtype (one spacing, 2^-7 bf16 / 2^-10 fp16 of the value)."""
+    from linatt_amd import _lib
+    from linatt_amd.kata_cache import state_rows
+    B, H, E = 1, 3, dk // M
+    print(f"\nsplit update/readout dk{dk} M{M} {variant} packed={packed} decay={decay} {dtype} T{T}", flush=True)
+    L = _lib.load()
+    var = (1 if variant == "sum" else 0) | (_lib.LINATT_KATA_PACKED_STATE if packed else 0)
+    P = state_rows(dk, M, variant, packed)
+    q, k = (gen((B, T, H, dk), 700 + dk + i, 0.5).to(dtype).cuda() for i in range(2))
+    v = gen((B, T, H, 64), 702 + dk).to(dtype).cuda()
+    c = -(gen((B, T, H), 703).abs() * 0.05).cumsum(1).cuda() if decay else None
+    o0, den0 = gen((B, T, H, 64), 706).to(dtype).cuda(), (gen((B, T, H), 707).abs() + 0.5).cuda()
+    code, sp, sc = _lib.dtype_code(dtype), _lib.stream_of(q), 1.0 / math.sqrt(E)
+    # the stored state of 40 earlier tokens (so psi(q) . z >= 0, as every score gives)
+    S0, z0 = torch.empty(B, H, P, 64, device="cuda"), torch.empty(B, H, P, device="cuda")
+    k0, v0 = gen((B, 40, H, dk), 704, 0.5).to(dtype).cuda(), gen((B, 40, H, 64), 705).to(dtype).cuda()
+    _lib.check("u", L.linatt_kata_gen_update(_lib.ptr(k0), _lib.ptr(v0), None, _lib.ptr(S0), _lib.ptr(z0), 0, B, 40, H,
+                                             dk, 64, M, var, sc, code, sp))
+    ru = L.linatt_kata_gen_update_workspace_bytes(B, T, H, dk, M, var, code)
+    rr = L.linatt_kata_gen_readout_workspace_bytes(B, T, H, dk, M, var, code)
+    # a long call of every score splits; how short a call still does depends on the partials' size
+    assert ru > 0 or T <= 257
+    out = []
+    for split in (False, True):
+        S, z, o, den = S0.clone(), z0.clone(), o0.clone(), den0.clone()
+        P_ = _lib.ptr
+        if split:
+            wu, wr = (torch.empty(n, device="cuda", dtype=torch.uint8) if n else None for n in (ru, rr))
+            _lib.check("r", L.linatt_kata_gen_readout_split(P_(q), P_(c), P_(S), P_(z), P_(o), P_(den), P_(wr), rr, B, T,
+                                                            H, dk, 64, M, var, sc, 1e-6, code, sp))
+            _lib.check("u", L.linatt_kata_gen_update_split(P_(k), P_(v), P_(c), P_(S), P_(z), 1, P_(wu), ru, B, T, H, dk,
+                                                           64, M, var, sc, code, sp))
+        else:
+            _lib.check("r", L.linatt_kata_gen_readout(P_(q), P_(c), P_(S), P_(z), P_(o), P_(den), B, T, H, dk, 64, M,
+                                                      var, sc, 1e-6, code, sp))
+            _lib.check("u", L.linatt_kata_gen_update(P_(k), P_(v), P_(c), P_(S), P_(z), 1, B, T, H, dk, 64, M, var, sc,
+                                                     code, sp))
+        out.append((S, z, o, den))
+    torch.cuda.synchronize()
+    (S1, z1, o1, d1), (S2, z2, o2, d2) = out
+    # sum|terms| over the largest feature of any row: |psi| <= M scale max|k|^2
+    fmax = M * sc * k.float().abs().amax() ** 2
+    n = T + 66
+    tol = 2 * n * 2.0 ** -24 * (T * fmax * v.float().abs().amax() + S0.abs().amax())
+    assert (S1 - S2).abs().max() <= tol
+    assert (z1 - z2).abs().max() <= 2 * n * 2.0 ** -24 * (T * fmax + z0.abs().amax())
+    qf = M * sc * q.float().abs().amax() ** 2
+    nr = P + 66
+    den_tol = 2 * nr * 2.0 ** -24 * (2 * P * qf * z0.abs().amax() + den0.abs().amax())
+    assert (d1 - d2).abs().max() <= den_tol
+    spacing = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    num_tol = 2 * nr * 2.0 ** -24 * (2 * P * qf * S0.abs().amax() + (o0.float().abs() * den0[..., None]).amax())
+    o_tol = spacing * o1.float().abs() + ((num_tol + o1.float().abs() * den_tol) / d1[..., None])
+    assert ((o1.float() - o2.float()).abs() <= o_tol).all()
