@@ -58,6 +58,20 @@ int linatt_kata_fwd(const void* q, const void* k, const void* v, const float* c,
                     float* den, int B, int T, int HQ, int H, int dk, int dv, int num_groups,
                     float scale, int variant, int dtype, void* stream);
 
+/* linatt_kata_fwd with the key tiles of a launch that leaves CUs idle (few
+ * (batch, head) pairs) split over more workgroups, their float32 partial sums
+ * in the workspace and added in order by a second launch.  workspace: 16-byte
+ * aligned, at least linatt_kata_fwd_workspace_bytes bytes, 0 where no split
+ * pays (it may then be NULL; decay: whether c is given).  Same results as
+ * linatt_kata_fwd up to the float32 summation order (float16: and the row
+ * scale, which follows each piece's own maximum). */
+size_t linatt_kata_fwd_workspace_bytes(int B, int T, int HQ, int H, int dk, int dv, int num_groups,
+                                       int variant, int decay, int dtype);
+int linatt_kata_fwd_split(const void* q, const void* k, const void* v, const float* c, void* o,
+                          float* den, void* workspace, size_t workspace_bytes, int B, int T, int HQ,
+                          int H, int dk, int dv, int num_groups, float scale, int variant, int dtype,
+                          void* stream);
+
 /* Bytes of workspace linatt_kata_bwd needs: two (B, T, HQ) float32 arrays
  * (-<o, dO> and scale^2 / den per row) and, for LINATT_BFLOAT16, dO scaled by
  * scale^2 / den (B, T, HQ, dv_dim), which the dk/dv pass reads instead of dO.

@@ -38,6 +38,8 @@ SIGNATURES = {
     "linatt_last_error": (ctypes.c_char_p, []),
     "linatt_kata_supported": (_i, [_i, _i, _i, _i, _i, _i]),
     "linatt_kata_fwd": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _vp]),
+    "linatt_kata_fwd_workspace_bytes": (_sz, [_i] * 10),
+    "linatt_kata_fwd_split": (_i, [_vp] * 7 + [_sz] + [_i] * 7 + [_f, _i, _i, _vp]),
     "linatt_kata_bwd_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "linatt_kata_bwd": (_i, [_vp] * 10 + [_i] * 7 + [_f, _i, _i, _vp]),
     "linatt_kata_bwd_dq": (_i, [_vp] * 10 + [_i] * 7 + [_f, _i, _i, _vp]),

@@ -7,6 +7,7 @@
 #include "linatt_hip.h"
 #include "delta_kernels.h"
 #include "kata_kernels.h"
+#include "kata_split.h"
 #include "misc_kernels.h"
 
 namespace {
@@ -210,28 +211,68 @@ int linatt_kata_supported(int dtype, int dk, int dv, int num_groups, int variant
   return compiled(dtype, dk, dv, num_groups) ? 1 : 0;
 }
 
-int linatt_kata_fwd(const void* q, const void* k, const void* v, const float* c, void* o,
-                    float* den, int B, int T, int HQ, int H, int dk, int dv, int num_groups,
-                    float scale, int variant, int dtype, void* stream) {
+// tiles per workgroup of a split forward (0: unsplit)
+static int fwd_split(int B, int T, int HQ, int dk, int M, int variant, bool decay, int dtype) {
+  return kata_fwd_split((int64_t)B * HQ, T,
+                        kata_fwd_tile_time(elt_bytes(dtype), dtype == LINATT_FLOAT16, dk, M,
+                                           variant == LINATT_KATA_SUM, decay));
+}
+
+static int kata_fwd_entry(const char* fn, const void* q, const void* k, const void* v, const float* c,
+                          void* o, float* den, bool split, void* ws, size_t ws_bytes, int B, int T,
+                          int HQ, int H, int dk, int dv, int num_groups, float scale, int variant,
+                          int dtype, void* stream) {
   g_last_error.clear();
   int st = check_common(B, T, HQ, H, dk, dv, num_groups, scale, variant, dtype);
   if (st) return st;
-  if (!q || !k || !v || !o || !den) return fail(LINATT_EINVAL, "linatt_kata_fwd: null tensor pointer");
+  if (!q || !k || !v || !o || !den) return fail(LINATT_EINVAL, std::string(fn) + ": null tensor pointer");
   if (c && variant != LINATT_KATA_CONCAT)
-    return fail(LINATT_EUNSUPPORTED, "linatt_kata_fwd: decay is only defined for the concat score");
+    return fail(LINATT_EUNSUPPORTED, std::string(fn) + ": decay is only defined for the concat score");
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
-    return fail(LINATT_EINVAL, "linatt_kata_fwd: q, k, v, o must be 16-byte aligned");
+    return fail(LINATT_EINVAL, std::string(fn) + ": q, k, v, o must be 16-byte aligned");
   KataArgs a{};
   a.q = q; a.k = k; a.v = v; a.c = c; a.o = o; a.den = den;
   a.B = B; a.T = T; a.HQ = HQ; a.H = H; a.DK = dk; a.DV = dv; a.M = num_groups; a.scale = scale;
+  if (split && compiled(dtype, dk, dv, num_groups)) {
+    a.split = fwd_split(B, T, HQ, dk, num_groups, variant, c != nullptr, dtype);
+    if (a.split) {
+      if (!ws || ws_bytes < kata_fwd_part_bytes((int64_t)B * HQ, T, a.split))
+        return fail(LINATT_EINVAL, std::string(fn) + ": workspace smaller than linatt_kata_fwd_workspace_bytes");
+      if (!aligned16(ws)) return fail(LINATT_EINVAL, std::string(fn) + ": workspace must be 16-byte aligned");
+      a.part = (float*)ws;
+    }
+  }
   bool found = false;
   hipError_t e = dispatch_fwd(a, dtype, variant, c != nullptr, (hipStream_t)stream, &found);
   if (!found)
-    return fail(LINATT_EUNSUPPORTED, "linatt_kata_fwd: no kernel compiled for " +
+    return fail(LINATT_EUNSUPPORTED, std::string(fn) + ": no kernel compiled for " +
                                          shape_str(B, T, HQ, H, dk, dv, num_groups));
   if (e != hipSuccess)
-    return fail(LINATT_ELAUNCH, std::string("linatt_kata_fwd: launch failed: ") + hipGetErrorString(e));
+    return fail(LINATT_ELAUNCH, std::string(fn) + ": launch failed: " + hipGetErrorString(e));
   return LINATT_OK;
+}
+
+int linatt_kata_fwd(const void* q, const void* k, const void* v, const float* c, void* o,
+                    float* den, int B, int T, int HQ, int H, int dk, int dv, int num_groups,
+                    float scale, int variant, int dtype, void* stream) {
+  return kata_fwd_entry("linatt_kata_fwd", q, k, v, c, o, den, false, nullptr, 0, B, T, HQ, H, dk, dv, num_groups,
+                        scale, variant, dtype, stream);
+}
+
+size_t linatt_kata_fwd_workspace_bytes(int B, int T, int HQ, int H, int dk, int dv, int num_groups,
+                                       int variant, int decay, int dtype) {
+  if (check_common(B, T, HQ, H, dk, dv, num_groups, 1.f, variant, dtype) || !compiled(dtype, dk, dv, num_groups))
+    return 0;
+  const int L = fwd_split(B, T, HQ, dk, num_groups, variant, decay != 0, dtype);
+  return L ? kata_fwd_part_bytes((int64_t)B * HQ, T, L) : 0;
+}
+
+int linatt_kata_fwd_split(const void* q, const void* k, const void* v, const float* c, void* o,
+                          float* den, void* workspace, size_t workspace_bytes, int B, int T, int HQ,
+                          int H, int dk, int dv, int num_groups, float scale, int variant, int dtype,
+                          void* stream) {
+  return kata_fwd_entry("linatt_kata_fwd_split", q, k, v, c, o, den, true, workspace, workspace_bytes, B, T, HQ, H,
+                        dk, dv, num_groups, scale, variant, dtype, stream);
 }
 
 size_t linatt_kata_bwd_workspace_bytes(int B, int T, int HQ, int dv_dim, int dtype) {

@@ -1095,7 +1095,7 @@ hipError_t launch_kata_bwd(const KataArgs& a, int parts, hipStream_t stream) {
       const int nbh = a.B * a.HQ;
       if constexpr (kTiles)
       {
-        const OutNorm on{a.nw, const_cast<void*>(a.dy), a.rstd, a.nw_part, a.eps, nullptr};
+        const OutNorm on{a.nw, const_cast<void*>(a.dy), a.rstd, a.nw_part, a.eps, nullptr, 0};
         auto go = [&](auto onorm) {
           kata_bwd_dq_tile_kernel<T, DK, DV, M, SUM, DECAY, decltype(onorm)::value>
               <<<dim3(nqt * nbh), dim3(256), 0, stream>>>(

@@ -25,14 +25,65 @@
 // goes back into the P.V product without leaving registers.
 #include "common.h"
 #include "kata_kernels.h"
+#include "kata_split.h"
 
 namespace linatt {
 
-template <typename T, int DK, int DV, int M, bool SUM, bool DECAY>
+// One piece's unnormalised sums of a wave's 32 queries, in register order (lane
+// l's 16 bytes i at 256 i + 4 l: whole 1 KiB runs per store, and the finish
+// kernel loads them back the same way; rows of o order instead scattered each
+// store over 32 rows and cost 10 to 25 us a call).  f undoes the fp16 row scale.
+template <int DV>
+__device__ __forceinline__ void store_fwd_partial(float* p, const f32x16 (&oacc)[DV / 32], float dsum, float f, int lane) {
+  static_assert(DV == 64, "32 x 64 blocks");
+#pragma unroll
+  for (int db = 0; db < 2; ++db)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<f32x4*>(p + 256 * (4 * db + i) + 4 * lane) =
+          f32x4{oacc[db][4 * i] * f, oacc[db][4 * i + 1] * f, oacc[db][4 * i + 2] * f, oacc[db][4 * i + 3] * f};
+  p[2048 + lane] = dsum * f;
+}
+// block `blk` (32 queries) of head bh, piece `piece`
+__host__ __device__ inline int64_t fwd_part_offset(int piece, int nbh, int bh, int nqt, int blk) {
+  return (((int64_t)piece * nbh + bh) * (4 * nqt) + blk) * kFwdPart;
+}
+
+// The split launch's outputs where the key list was cut: a wave per 32
+// queries, the pieces added in order.
+template <typename T>
+__global__ __launch_bounds__(256) void kata_fwd_split_finish_kernel(const float* __restrict__ part, T* __restrict__ o,
+                                                                    float* __restrict__ den, int Tn, int HQ, int nqt,
+                                                                    int nbh, float scale2, int split) {
+  const int lane = threadIdx.x & 63, cl = lane & 31, hh = lane >> 5;
+  const int qt = blockIdx.x % nqt, bh = blockIdx.x / nqt, w = wave_id();
+  const int pieces = split_pieces(kata_key_tiles(qt, Tn), split);
+  if (pieces == 1) return;
+  f32x4 x[8] = {};
+  float dsum = 0.f;
+#pragma unroll 2
+  for (int i = 0; i < pieces; ++i) {
+    const float* p = part + fwd_part_offset(i, nbh, bh, nqt, 4 * qt + w);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] += *reinterpret_cast<const f32x4*>(p + 256 * e + 4 * lane);
+    dsum += p[2048 + lane];
+  }
+  const int tl = 128 * qt + 32 * w + cl;
+  if (tl >= Tn) return;
+  const float inv = dsum > 0.f ? 1.f / dsum : 1.f;
+  const int64_t row = ((int64_t)(bh / HQ) * Tn + tl) * HQ + bh % HQ;
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    st4<T>(o + row * 64 + 8 * e + 4 * hh, to4<T>(x[e][0] * inv, x[e][1] * inv, x[e][2] * inv, x[e][3] * inv));
+  if (hh == 0) den[row] = dsum * scale2;
+}
+
+// SPLIT: the workgroup's share of a split launch (kata_split.h)
+template <typename T, int DK, int DV, int M, bool SUM, bool DECAY, bool SPLIT>
 __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void kata_fwd_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const float* __restrict__ c, T* __restrict__ o, float* __restrict__ den,
-    int Tn, int HQ, int H, float scale2, int nqt, int nbh) {
+    int Tn, int HQ, int H, float scale2, int nqt, int nbh, int split, float* __restrict__ part) {
   constexpr int E = DK / M;
   constexpr int KE = E / 16;           // 16-wide k-steps per group
   constexpr int KP = DK + (sizeof(T) == 2 ? 8 : 4);   // K tile pitch
@@ -45,7 +96,15 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void kata_fwd_kernel(
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
   const int cl = lane & 31, hh = lane >> 5;
   int qt, bh;
-  map_block(blockIdx.x, nqt, nbh, qt, bh, true);
+  SplitRun run{};
+  if constexpr (SPLIT) {
+    int item;
+    map_block(blockIdx.x, gridDim.x / nbh, nbh, item, bh, false);
+    run = kata_fwd_run(item, nqt, Tn, split);
+    qt = run.tile;
+  } else {
+    map_block(blockIdx.x, nqt, nbh, qt, bh, true);
+  }
   const int b = bh / HQ, hq = bh % HQ;
   const int G = HQ / H, h = hq / G;
   const int t0 = qt * 128;
@@ -77,8 +136,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void kata_fwd_kernel(
   float pe = 1.f, mrun = 0.f;
 
   const int s_end = min(t0 + 128, Tn);
-  const int nst = (s_end + 63) / 64;
-  for (int st = 0; st < nst; ++st) {
+  const int st0 = SPLIT ? run.lo : 0, nst = SPLIT ? run.hi : (s_end + 63) / 64;
+  for (int st = st0; st < nst; ++st) {
     const int s0 = st * 64;
     __syncthreads();
     load_tile64<T, DK, KP, 1, true, false>(kb, s0, Tn, ks, Ks, nullptr, tid);
@@ -175,6 +234,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void kata_fwd_kernel(
   }
 
   const float dsum = dpart + __shfl_xor(dpart, 32);
+  if constexpr (SPLIT) {
+    if (run.pieces > 1) {
+      store_fwd_partial<DV>(part + fwd_part_offset(run.piece, nbh, bh, nqt, 4 * qt + w), oacc, dsum, 1.f / pe, lane);
+      return;
+    }
+  }
   if (tl < Tn) {
     const float inv = dsum > 0.f ? 1.f / dsum : 1.f;
     T* orow = o + (((int64_t)b * Tn + tl) * HQ + hq) * DV;
@@ -199,8 +264,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void kata_fwd_kernel(
 // fixed for the kernel plus an immediate, and full tiles are copied from a
 // scalar base: the VALU, which bounds this kernel, only does the math.
 // EPI: 0 writes o; 1 also the output RMSNorm's y and rstd; 2 the float32
-// numerator o den instead of o (compile-time, so each variant carries only
-// its own epilogue).  Three waves per SIMD at dk = 64 (at most 168 VGPRs;
+// numerator o den instead of o; 3 the workgroup's share of a split launch
+// (kata_split.h: its run of key tiles, and partial rows where the list was
+// cut) (compile-time, so each variant carries only its own epilogue).  Three waves per SIMD at dk = 64 (at most 168 VGPRs;
 // the compiler otherwise lets some variants grow just past it)
 template <typename T, int DK, int DV, int M, bool SUM, bool DECAY, int EPI>
 __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void kata_fwd_tile_kernel(
@@ -219,7 +285,15 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void kata_fwd_tile_kernel(
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
   const int cl = lane & 31, hh = lane >> 5;
   int qt, bh;
-  map_block(blockIdx.x, nqt, nbh, qt, bh, true);
+  SplitRun run{};
+  if constexpr (EPI == 3) {
+    int item;
+    map_block(blockIdx.x, gridDim.x / nbh, nbh, item, bh, false);
+    run = kata_fwd_run(item, nqt, Tn, on.split);
+    qt = run.tile;
+  } else {
+    map_block(blockIdx.x, nqt, nbh, qt, bh, true);
+  }
   const int b = bh / HQ, hq = bh % HQ;
   const int G = HQ / H, h = hq / G;
   const int t0 = qt * 128;
@@ -246,7 +320,8 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void kata_fwd_tile_kernel(
   float pe = 1.f, mrun = 0.f;
 
   const int s_end = min(t0 + 128, Tn);
-  const int nst = (s_end + 63) / 64;
+  // key tiles [st0, nst), ring slots in turn from st0 on
+  const int st0 = EPI == 3 ? run.lo : 0, nst = EPI == 3 ? run.hi : (s_end + 63) / 64;
   // tile st: 8 KiB of K and 8 KiB of V, copies 2w and 2w + 1 of each by wave w
   // (full tiles: scalar base + these per-lane offsets)
   unsigned ko[2], vo[2];
@@ -432,10 +507,10 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void kata_fwd_tile_kernel(
   };
 
   vm_drain();  // q (and c) of this wave's queries are in registers
-  issue(0, IntC<0>{});
-  if (nst > 1) issue(1, IntC<1>{});
+  issue(st0, IntC<0>{});
+  if (st0 + 1 < nst) issue(st0 + 1, IntC<1>{});
   constexpr bool kPlain = !SUM && !DECAY && !kRescale;
-  int st = 0;
+  int st = st0;
   if constexpr (kPlain) {
     // tiles wholly before this workgroup's first query, then the rest
     const int nplain = min(t0 / 64, nst);
@@ -448,7 +523,7 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void kata_fwd_tile_kernel(
     if (st < nplain) step_plain(st++, IntC<1>{});
   }
   for (; st < nst; ++st) {
-    switch (st % NB) {
+    switch ((st - st0) % NB) {
       case 0: step(st, IntC<0>{}); break;
       case 1: step(st, IntC<1>{}); break;
       default: step(st, IntC<2>{}); break;
@@ -456,6 +531,13 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void kata_fwd_tile_kernel(
   }
 
   const float dsum = dpart + __shfl_xor(dpart, 32);
+  if constexpr (EPI == 3) {
+    if (run.pieces > 1) {
+      store_fwd_partial<DV>(on.part + fwd_part_offset(run.piece, nbh, bh, nqt, 4 * qt + w), oacc, dsum, 1.f / pe,
+                            lane);
+      return;
+    }
+  }
   const float inv = dsum > 0.f ? 1.f / dsum : 1.f;
   // this lane's 32 elements of its query's output row (dims 32 db + 8 i +
   // 4 hh + r), rounded to T as stored
@@ -526,8 +608,15 @@ hipError_t launch_kata_fwd(const KataArgs& a, hipStream_t stream) {
     const int nqt = (a.T + 127) / 128;
     const int nbh = a.B * a.HQ;
     dim3 grid(nqt * nbh), block(256);
+    if (a.split && (a.y || a.num32)) return hipErrorInvalidValue;  // o only
+    if (a.split) grid.x = kata_fwd_items(a.T, a.split) * nbh;
+    auto finish = [&]() {
+      if (!a.split) return;
+      kata_fwd_split_finish_kernel<T><<<dim3(nqt * nbh), block, 0, stream>>>(
+          a.part, (T*)a.o, a.den, a.T, a.HQ, nqt, nbh, a.scale * a.scale, a.split);
+    };
     if constexpr (sizeof(T) == 2 && (DK == 64 || DK == 128) && DV == 64) {
-      const OutNorm on{a.nw, a.y, a.rstd, nullptr, a.eps, a.num32};
+      const OutNorm on{a.nw, a.y, a.rstd, a.part, a.eps, a.num32, a.split};
       auto go = [&](auto epi) {
         kata_fwd_tile_kernel<T, DK, DV, M, SUM, DECAY, decltype(epi)::value><<<grid, block, 0, stream>>>(
             (const T*)a.q, (const T*)a.k, (const T*)a.v, a.c, (T*)a.o, a.den, a.T, a.HQ, a.H,
@@ -536,14 +625,20 @@ hipError_t launch_kata_fwd(const KataArgs& a, hipStream_t stream) {
       if (a.y && a.num32) return hipErrorInvalidValue;
       if (a.y) go(IntC<1>{});
       else if (a.num32) go(IntC<2>{});
+      else if (a.split) go(IntC<3>{});
       else go(IntC<0>{});
     } else {
       // the output norm and the float32 numerator are tile-kernel options
       if (a.y || a.num32) return hipErrorInvalidValue;
-      kata_fwd_kernel<T, DK, DV, M, SUM, DECAY><<<grid, block, 0, stream>>>(
-          (const T*)a.q, (const T*)a.k, (const T*)a.v, a.c, (T*)a.o, a.den, a.T, a.HQ, a.H,
-          a.scale * a.scale, nqt, nbh);
+      auto go = [&](auto sp) {
+        kata_fwd_kernel<T, DK, DV, M, SUM, DECAY, decltype(sp)::value><<<grid, block, 0, stream>>>(
+            (const T*)a.q, (const T*)a.k, (const T*)a.v, a.c, (T*)a.o, a.den, a.T, a.HQ, a.H,
+            a.scale * a.scale, nqt, nbh, a.split, a.part);
+      };
+      if (a.split) go(BoolC<true>{});
+      else go(BoolC<false>{});
     }
+    finish();
     return hipGetLastError();
   }
 }

@@ -41,6 +41,10 @@ struct KataArgs {
   // numerator num = o den = sum_s A[t,s] v_s is written here in float32
   // instead of o (o may then be null)
   float* num32;
+  // forward: tiles per workgroup of a split launch (kata_split.h; 0: unsplit)
+  // and its partial blocks (pieces, B HQ, 4 ceil(T / 128), kFwdPart) float32
+  int split;
+  float* part;
 };
 
 // The output-norm arguments of the tile kernels (a kernel argument struct).
@@ -51,6 +55,7 @@ struct OutNorm {
   float* part;    // backward: weight-gradient partials, or null
   float eps;
   float* num;     // forward: float32 numerator instead of o, or null
+  int split;      // forward: tiles per workgroup of a split launch, whose partial blocks go to `part`
 };
 
 template <typename T, int DK, int DV, int M, bool SUM, bool DECAY>

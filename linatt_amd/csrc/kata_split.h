@@ -1,0 +1,124 @@
+// Work split of the KATA attention passes for launches with few workgroups.
+//
+// Unsplit, one workgroup walks every key tile of its 128 queries (forward),
+// a serial chain of up to T / 64 tiles: at B1 H12 T3001 that is 288 chains
+// on 256 CUs, the longest 47 tiles.  The score has no softmax maximum, so the
+// sums of disjoint key ranges simply add: the split gives every tile list
+// longer than L to several workgroups of at most L tiles each, whose float32
+// partial sums a second launch adds in order.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace linatt {
+
+// pieces of a list of n tiles cut into runs of at most L (all but the last
+// equally long, none empty)
+__host__ __device__ inline int split_pieces(int n, int L) { return (n + L - 1) / L; }
+
+// 64-key tiles of query tile qt (128 queries, causal)
+__host__ __device__ inline int kata_key_tiles(int qt, int T) {
+  const int s_end = 128 * qt + 128 < T ? 128 * qt + 128 : T;
+  return (s_end + 63) / 64;
+}
+inline int kata_fwd_items(int T, int L) {
+  int n = 0;
+  for (int qt = 0; qt < (T + 127) / 128; ++qt) n += split_pieces(kata_key_tiles(qt, T), L);
+  return n;
+}
+
+struct SplitRun {
+  int tile, piece, pieces, lo, hi;  // tiles [lo, hi) of list `tile`
+};
+// item j of a head's (list, piece) pairs, longest lists first
+__device__ __forceinline__ SplitRun kata_fwd_run(int j, int nqt, int T, int L) {
+  SplitRun r;
+  r.tile = nqt - 1;
+  int n = kata_key_tiles(r.tile, T);
+  r.pieces = split_pieces(n, L);
+  while (j >= r.pieces) {
+    j -= r.pieces;
+    --r.tile;
+    n = kata_key_tiles(r.tile, T);
+    r.pieces = split_pieces(n, L);
+  }
+  r.piece = j;
+  const int per = (n + r.pieces - 1) / r.pieces;
+  r.lo = j * per;
+  r.hi = r.lo + per < n ? r.lo + per : n;
+  return r;
+}
+
+// floats of a partial block of 32 queries: 32 x 64 sums, a den per lane
+constexpr int kFwdPart = 32 * 64 + 64;
+// most pieces of one list (the partial blocks reserved for it)
+constexpr int kMaxPieces = 16;
+
+// A workgroup's time per tile alone on its CU and with the CU full (slots / 256
+// workgroups sharing it).
+struct TileTime {
+  double solo_us, full_us;
+  int slots;
+};
+
+// Tiles per workgroup with the least modelled time, 0 to leave the launch
+// unsplit.  Modelled as the longer of the longest list at the solo rate and
+// the whole work over all slots at the full rate; for a split the rate of its
+// runs is 1.3 solo and half a run is left uneven at the end, and it adds 8 us
+// (the second launch, and the first tile's latency in every workgroup) and the
+// partial blocks written and read at 4.5 TB/s.  It has to win by a tenth.
+template <typename Lists>
+inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileTime& tt, double list_bytes) {
+  int64_t units = 0;
+  int longest = 0;
+  for (int i = 0; i < nlists; ++i) {
+    const int n = lists(i);
+    units += n;
+    if (n > longest) longest = n;
+  }
+  const double all = (double)(units * heads) * tt.full_us / tt.slots;
+  auto longer = [](double a, double b) { return a > b ? a : b; };
+  double best = 0.9 * longer(longest * tt.solo_us, all);
+  int L_best = 0;
+  for (int L = 1; L < longest; L = L < 4 ? L + 1 : L + L / 4) {
+    if (split_pieces(longest, L) > kMaxPieces) continue;
+    int64_t part = 0;
+    for (int i = 0; i < nlists; ++i) {
+      const int p = split_pieces(lists(i), L);
+      if (p > 1) part += p;
+    }
+    const double t = longer(1.3 * L * tt.solo_us, all + 0.5 * L * tt.solo_us) + 8. +
+                     (double)(part * heads) * list_bytes * (2. / 4.5e6);
+    if (t < best) {
+      best = t;
+      L_best = L;
+    }
+  }
+  return L_best;
+}
+
+// Forward, per 64-key tile of 128 queries (measured, B1 to B8, H = 12).  16-bit:
+// three workgroups per CU at dk = 64, two at dk = 128; fp16 adds the row
+// rescaling.  float32: 32 x 32 x 2 products, two workgroups per CU.
+// Unsplit -> split, us: float32 B1 H4 T512 48 -> 20; fp16 M = 2 B1 H12 T3001
+// 57 -> 40; bf16 B1 H12 T2048: sum M = 4 76 -> 40, decayed dk = 128 55 -> 33,
+// concat M = 4 28 -> 26.  Left unsplit: concat M = 4 at B2 T2048 (30 against 33),
+// B4 (39 against 51), M = 1 at B1 T1500 (18 against 19).
+inline TileTime kata_fwd_tile_time(int elt_bytes, bool fp16, int dk, int M, bool sum, bool decay) {
+  if (elt_bytes == 4) return {6., 14., 512};
+  double solo = sum && M > 1 ? (M == 2 ? 1.3 : 2.4) : 0.85;
+  if (dk == 128) solo *= 1.4;
+  if (decay) solo *= 1.4;
+  if (fp16) solo *= 1.4;
+  return dk == 128 ? TileTime{solo, 1.4 * solo, 512} : TileTime{solo, 2.2 * solo, 768};
+}
+inline int kata_fwd_split(int64_t BH, int T, const TileTime& tt) {
+  return best_split([&](int qt) { return kata_key_tiles(qt, T); }, BH, (T + 127) / 128, tt, 4. * kFwdPart * 4);
+}
+// partial blocks of a forward split by L, bytes
+inline size_t kata_fwd_part_bytes(int64_t BH, int T, int L) {
+  const int nqt = (T + 127) / 128;
+  return (size_t)split_pieces(kata_key_tiles(nqt - 1, T), L) * BH * 4 * nqt * kFwdPart * sizeof(float);
+}
+
+}  // namespace linatt

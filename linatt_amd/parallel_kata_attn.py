@@ -24,6 +24,7 @@ unsupported combinations raise, nothing falls back to PyTorch math.
 
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -83,11 +84,20 @@ def _fwd(q, k, v, num_groups, scale, variant, c=None):
         c = c.float().contiguous()
         assert c.shape == (B, T, HQ), f"c must be (B,T,HQ) = {(B, T, HQ)}, got {tuple(c.shape)}"
     L = _lib.load()
-    _lib.check("linatt_kata_fwd", L.linatt_kata_fwd(
-        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(c), _lib.ptr(o), _lib.ptr(den),
-        B, T, HQ, H, dk, dv, num_groups, float(scale), _VARIANT[variant],
-        _lib.dtype_code(v.dtype), _lib.stream_of(q)))
+    # a launch that leaves CUs idle splits its key tiles over more workgroups
+    shape = (B, T, HQ, H, dk, dv, num_groups)
+    code, var = _lib.dtype_code(v.dtype), _VARIANT[variant]
+    nws = _fwd_workspace_bytes(*shape, var, int(c is not None), code)
+    ws = torch.empty(nws, device=q.device, dtype=torch.uint8) if nws else None
+    _lib.check("linatt_kata_fwd_split", L.linatt_kata_fwd_split(
+        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(c), _lib.ptr(o), _lib.ptr(den), _lib.ptr(ws), nws,
+        *shape, float(scale), var, code, _lib.stream_of(q)))
     return o, den
+
+
+@functools.lru_cache(maxsize=256)
+def _fwd_workspace_bytes(*args):
+    return _lib.load().linatt_kata_fwd_workspace_bytes(*args)
 
 
 def _bwd(q, k, v, o, den, do, num_groups, scale, variant):
