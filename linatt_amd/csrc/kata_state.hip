@@ -642,6 +642,17 @@ __global__ __launch_bounds__(256) void kata_decode_kernel(KataDecodeArgs a) {
   // this workgroup's rows [p_lo, p_hi) of the a.nsplit runs (multiples of 16)
   const int run = ((NR + a.nsplit - 1) / a.nsplit + 15) & ~15;
   const int p_lo = sp * run, p_hi = min(NR, p_lo + run);
+  const int c4 = tid & 15, r = tid >> 4;
+  float* S = a.S + (size_t)bh * NR * DV;
+  float* z = a.z + (size_t)bh * NR;
+  float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+  float zs = 0.f;
+  auto load = [&](int p) __attribute__((always_inline)) {
+    if (p >= p_hi) return;
+    x = *reinterpret_cast<const float4*>(S + (size_t)p * DV + 4 * c4);
+    if (c4 == 0) zs = z[p];
+  };
+  load(p_lo + r);
   if (tid < DK) {
     qs[tid] = (float)((const T*)a.q)[(size_t)bh * DK + tid];
     ks[tid] = (float)((const T*)a.k)[(size_t)bh * DK + tid];
@@ -659,13 +670,11 @@ __global__ __launch_bounds__(256) void kata_decode_kernel(KataDecodeArgs a) {
     }
   }
   __syncthreads();
-  const int c4 = tid & 15, r = tid >> 4;
   const float4 vv = *reinterpret_cast<const float4*>(vs + 4 * c4);
   float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
   float dacc = 0.f;
-  float* S = a.S + (size_t)bh * NR * DV;
-  float* z = a.z + (size_t)bh * NR;
   for (int p = p_lo + r; p < p_hi; p += 16) {
+    if (p != p_lo + r) load(p);
     int ia, ib;
     float wq = a.scale;
     if constexpr (TRI) {
@@ -680,13 +689,11 @@ __global__ __launch_bounds__(256) void kata_decode_kernel(KataDecodeArgs a) {
     }
     const float pk = a.scale * ks[ia] * ks[ib];
     const float pq = wq * qs[ia] * qs[ib];
-    float4* sp = reinterpret_cast<float4*>(S + (size_t)p * DV + 4 * c4);
-    float4 x = *sp;
     x.x += pk * vv.x; x.y += pk * vv.y; x.z += pk * vv.z; x.w += pk * vv.w;
-    *sp = x;
+    *reinterpret_cast<float4*>(S + (size_t)p * DV + 4 * c4) = x;
     num.x += pq * x.x; num.y += pq * x.y; num.z += pq * x.z; num.w += pq * x.w;
     if (c4 == 0) {
-      const float zz = z[p] + pk;
+      const float zz = zs + pk;
       z[p] = zz;
       dacc += pq * zz;
     }
