@@ -773,8 +773,12 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
   __shared__ __attribute__((aligned(16))) float Dl[NB][64];  // -delta
   __shared__ __attribute__((aligned(16))) float Pd[NB][64];  // scale^2 / den
   __shared__ __attribute__((aligned(16))) float Ct[NB][64];
-  // this wave's k and v rows as MFMA B operands (lane l: 16 bytes per k-step)
-  __shared__ __attribute__((aligned(16))) u32x4 KVop[NW][(DK + DV) / 16][64];
+  // bf16 dk = 64 without decay: the pipelined body for unmasked tiles (below),
+  // and this wave's k and v rows (MFMA B operands, 16 bytes per lane and
+  // k-step) in registers; the other variants have no 32 registers left and
+  // keep the operands in LDS
+  constexpr bool kPipe = __is_same(T, __bf16) && !DECAY && DK == 64;
+  __shared__ __attribute__((aligned(16))) u32x4 KVop[kPipe ? 1 : NW][kPipe ? 1 : (DK + DV) / 16][kPipe ? 1 : 64];
 
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
   const int cl = lane & 31, hh = lane >> 5;
@@ -790,14 +794,23 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
   const int64_t qs = (int64_t)HQ * DK, os = (int64_t)HQ * DV;
   const int64_t krow = ((int64_t)b * Tn + sl) * H + h;
 
+  u32x4 kvreg[kPipe ? (DK + DV) / 16 : 1];
+  auto kv_put = [&](int kk, v8_t<T> x) __attribute__((always_inline)) {
+    if constexpr (kPipe) kvreg[kk] = __builtin_bit_cast(u32x4, x);
+    else KVop[w][kk][lane] = __builtin_bit_cast(u32x4, x);
+  };
+  auto kv_get = [&](int kk) __attribute__((always_inline)) {
+    if constexpr (kPipe) return __builtin_bit_cast(v8_t<T>, kvreg[kk]);
+    else return __builtin_bit_cast(v8_t<T>, KVop[w][kk][lane]);
+  };
 #pragma unroll
   for (int kk = 0; kk < DK / 16; ++kk)
-    KVop[w][kk][lane] = __builtin_bit_cast(u32x4, svalid ? ld8<T>(k + krow * DK + 16 * kk + 8 * hh) : zero8<T>());
+    kv_put(kk, svalid ? ld8<T>(k + krow * DK + 16 * kk + 8 * hh) : zero8<T>());
 #pragma unroll
   for (int kk = 0; kk < DV / 16; ++kk)
-    KVop[w][DK / 16 + kk][lane] = __builtin_bit_cast(u32x4, svalid ? ld8<T>(v + krow * DV + 16 * kk + 8 * hh) : zero8<T>());
-  auto kop = [&](int kk) __attribute__((always_inline)) { return __builtin_bit_cast(v8_t<T>, KVop[w][kk][lane]); };
-  auto vop = [&](int kk) __attribute__((always_inline)) { return __builtin_bit_cast(v8_t<T>, KVop[w][DK / 16 + kk][lane]); };
+    kv_put(DK / 16 + kk, svalid ? ld8<T>(v + krow * DV + 16 * kk + 8 * hh) : zero8<T>());
+  auto kop = [&](int kk) __attribute__((always_inline)) { return kv_get(kk); };
+  auto vop = [&](int kk) __attribute__((always_inline)) { return kv_get(DK / 16 + kk); };
 
   // 16-wide groups (E = 16): dK_g^T (16 x 32 keys) by two 16x16x32 products
   // per group and query block, B operands from da by one lane swap per
@@ -1033,13 +1046,130 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
       }
     }
   };
+  // unmasked tiles, software-pipelined over the tile's 2 NU (block, group pair)
+  // units
+  auto tile_pipe = [&](int n) __attribute__((always_inline)) {
+    constexpr int NU = SUM ? M * M : M;
+    const int buf = n % NB;
+    vm_wait_barrier_n(0);
+    if (n + 1 < ntiles) {
+      issue(n + 1, 1 - buf);
+      load_rows(n + 1, 1 - buf);
+    }
+    const int t0 = 64 * (tt0 + n % nq);
+    if (t0 + 63 < sw || sw >= Tn) return;
+    const T* Qs = Qb[buf];
+    const T* Os = Ob[buf];
+    auto gi_of = [](int U) { return SUM ? (U % NU) / M : U % NU; };
+    auto gk_of = [](int U) { return SUM ? (U % NU) % M : U % NU; };
+    v8_t<T> qo2[2][KE], ko2[2][KE];
+    auto sread = [&](int U) __attribute__((always_inline)) {
+#pragma unroll
+      for (int kk = 0; kk < KE; ++kk) {
+        qo2[U & 1][kk] = wtile_ld8<T>(Qs + 2048 * (U / NU), cl, gi_of(U) * E + 16 * kk + 8 * hh);
+        ko2[U & 1][kk] = kop(gk_of(U) * KE + kk);
+      }
+    };
+    auto score = [&](int U) __attribute__((always_inline)) {
+      f32x16 r{};
+#pragma unroll
+      for (int kk = 0; kk < KE; ++kk) r = mma(qo2[U & 1][kk], ko2[U & 1][kk], r);
+      return r;
+    };
+    auto xchain = [&](int mb) __attribute__((always_inline)) {
+      f32x16 x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 d4 = *reinterpret_cast<const f32x4*>(&Dl[buf][32 * mb + 8 * i + 4 * hh]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[4 * i + r] = d4[r];
+      }
+#pragma unroll
+      for (int kk = 0; kk < DV / 16; ++kk)
+        x = mma(tile_ld8<T>(Os + 2048 * mb, cl, 16 * kk + 8 * hh), vop(kk), x);
+      return x;
+    };
+    f32x16 x0 = xchain(0), x1, A;
+    sread(0);
+    sread(1);
+    f32x16 rc = score(0);
+    v8_t<T> b0, b1, pp[2];
+    v8_t<T> qa[k16 ? 1 : (E / 32) * 2];
+    __builtin_amdgcn_sched_barrier(0);
+    auto dkread = [&](int U) __attribute__((always_inline)) {
+      const int mb = U / NU, gi = gi_of(U), gk = gk_of(U);
+      if constexpr (k16) {
+        qa[0] = tile_tr8_16<T>(Qs, 32 * mb, 16 * gi, lane);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int rb = 0; rb < E / 32; ++rb) qa[j * (E / 32) + rb] = qt_op(Qs, mb, gi, gk, gk * E / 32 + rb, j);
+      }
+    };
+    auto dkmma = [&](int U) __attribute__((always_inline)) {
+      const int gk = gk_of(U);
+      if constexpr (k16) {
+        dk16[gk][0] = mma16(qa[0], b0, dk16[gk][0]);
+        dk16[gk][1] = mma16(qa[0], b1, dk16[gk][1]);
+      } else {
+#pragma unroll
+        for (int rb = 0; rb < E / 32; ++rb) {
+          dka[gk * E / 32 + rb] = mma(qa[rb], b0, dka[gk * E / 32 + rb]);
+          dka[gk * E / 32 + rb] = mma(qa[E / 32 + rb], b1, dka[gk * E / 32 + rb]);
+        }
+      }
+    };
+    auto dvmma = [&](int mb, int i) __attribute__((always_inline)) {
+      dva[i & 1] = mma(tile_tr8<T>(Os, 32 * mb, 32 * (i & 1), i >> 1, lane), pp[i >> 1], dva[i & 1]);
+    };
+#pragma unroll
+    for (int U = 0; U < 2 * NU; ++U) {
+      const int mb = U / NU, u = U % NU;
+      f32x16 rn;
+      if (U + 1 < 2 * NU) rn = score(U + 1);
+      if (U > 0) dkmma(U - 1);
+      if (mb == 1) {
+        // block 0's dV products spread over block 1's first units
+        constexpr int PER = NU >= 4 ? 1 : 4 / NU;
+        if (u * PER < 4) {
+#pragma unroll
+          for (int i = 0; i < PER; ++i) dvmma(0, u * PER + i);
+        }
+      }
+      if (mb == 0 && u == (NU > 1 ? NU - 2 : 0)) x1 = xchain(1);
+      if (U + 2 < 2 * NU) sread(U + 2);
+      dkread(U);
+      const f32x16 da = rc * (mb == 0 ? x0 : x1);
+      if constexpr (k16) {
+        c_to_b16x2<T>(da, b0, b1);
+      } else {
+        b0 = c_to_b<T>(da, 0);
+        b1 = c_to_b<T>(da, 1);
+      }
+      if (u == 0) A = rc * rc; else A += rc * rc;
+      if (u == NU - 1) {
+        pp[0] = c_to_b<T>(A, 0);
+        pp[1] = c_to_b<T>(A, 1);
+      }
+      rc = rn;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    dkmma(2 * NU - 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dvmma(1, i);
+  };
   // per query head: the diagonal tiles, the tiles wholly inside T, the ragged rest
   const int nfull = Tn / 64 - tt0;
   for (int hi = 0; hi < G; ++hi) {
     const int nb = hi * nq;
     int i = 0;
     for (; i < nq && i < NW / 2; ++i) tile(nb + i, BoolC<true>{});
-    for (; i < nfull; ++i) tile(nb + i, BoolC<false>{});
+    if constexpr (kPipe) {
+      for (; i < nfull; ++i) tile_pipe(nb + i);
+    } else {
+      for (; i < nfull; ++i) tile(nb + i, BoolC<false>{});
+    }
     for (; i < nq; ++i) tile(nb + i, BoolC<true>{});
   }
 
