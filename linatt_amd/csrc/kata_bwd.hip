@@ -644,32 +644,54 @@ __global__ __launch_bounds__(256, 2) void kata_bwd_dq_tile_kernel(
           }
         }
         f32x16 au{};
+        constexpr int NU = SUM ? M * M : M;  // (query group, key group) pairs
+        auto gi_of = [](int u) { return SUM ? u / M : u; };
+        auto gk_of = [](int u) { return SUM ? u % M : u; };
+        auto score = [&](int u) __attribute__((always_inline)) {
+          f32x16 r{};
 #pragma unroll
-        for (int gi = 0; gi < M; ++gi) {
+          for (int kk = 0; kk < KE; ++kk)
+            r = mma(wtile_ld8<T>(Ks, 32 * sb + cl, gk_of(u) * E + 16 * kk + 8 * hh), qop[gi_of(u) * KE + kk], r);
+          return r;
+        };
+        // dk = 128, sum and decayed scores (two waves per SIMD, four-step
+        // score chains): the next pair's score is issued under this pair's
+        // VALU work and products, and the fence keeps the compiler from
+        // interleaving further pairs, which spills (B8 H12 T2048: decayed
+        // 230 -> 205 us, sum 223 -> 213; concat 143 -> 145, left alone).  At
+        // dk = 64 the 16 registers more cost the third wave per SIMD (M = 4:
+        // 101 -> 110)
+        constexpr bool kAhead = DK == 128 && (SUM || DECAY);
+        f32x16 r, rn;
+        if constexpr (kAhead) r = score(0);
 #pragma unroll
-          for (int gj = 0; gj < (SUM ? M : 1); ++gj) {
-            const int gk = SUM ? gj : gi;
-            f32x16 r{};
+        for (int u = 0; u < NU; ++u) {
+          const int gi = gi_of(u), gk = gk_of(u);
+          if constexpr (kAhead) {
+            if (u + 1 < NU) rn = score(u + 1);
+          } else {
+            r = score(u);
+          }
+          if constexpr (DECAY) au += r * r;
+          const f32x16 da = r * x;
+          if constexpr (k16) {
+            v8_t<T> b0, b1;
+            c_to_b16x2<T>(da, b0, b1);
+            const v8_t<T> ka = tile_tr8_16<T>(Ks, 32 * sb, 16 * gk, lane);
+            acc16[gi][0] = mma16(ka, b0, acc16[gi][0]);
+            acc16[gi][1] = mma16(ka, b1, acc16[gi][1]);
+          } else {
 #pragma unroll
-            for (int kk = 0; kk < KE; ++kk)
-              r = mma(wtile_ld8<T>(Ks, 32 * sb + cl, gk * E + 16 * kk + 8 * hh), qop[gi * KE + kk], r);
-            if constexpr (DECAY) au += r * r;
-            const f32x16 da = r * x;
-            if constexpr (k16) {
-              v8_t<T> b0, b1;
-              c_to_b16x2<T>(da, b0, b1);
-              const v8_t<T> ka = tile_tr8_16<T>(Ks, 32 * sb, 16 * gk, lane);
-              acc16[gi][0] = mma16(ka, b0, acc16[gi][0]);
-              acc16[gi][1] = mma16(ka, b1, acc16[gi][1]);
-            } else {
+            for (int j = 0; j < 2; ++j) {
+              const v8_t<T> bop = c_to_b<T>(da, j);
 #pragma unroll
-              for (int j = 0; j < 2; ++j) {
-                const v8_t<T> bop = c_to_b<T>(da, j);
-#pragma unroll
-                for (int rb = (gi * E) / 32; rb <= ((gi + 1) * E - 1) / 32; ++rb)
-                  acc[rb] = mma(kt_op(Ks, sb, gi, gk, rb, j), bop, acc[rb]);
-              }
+              for (int rb = (gi * E) / 32; rb <= ((gi + 1) * E - 1) / 32; ++rb)
+                acc[rb] = mma(kt_op(Ks, sb, gi, gk, rb, j), bop, acc[rb]);
             }
+          }
+          if constexpr (kAhead) {
+            r = rn;
+            if (u + 1 < NU) __builtin_amdgcn_sched_barrier(0);
           }
         }
         if constexpr (DECAY) {
@@ -1047,7 +1069,14 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
     }
   };
   // unmasked tiles, software-pipelined over the tile's 2 NU (block, group pair)
-  // units
+  // units: the next unit's score and the previous one's dK product are issued
+  // under this unit's VALU work, block 1's x chain under block 0's last units
+  // and block 0's dV products under block 1's first; the fences keep that
+  // order.  VALU-bound with the MFMA issue (204 VALU and 20 MFMA a block at M =
+  // 4, most of which the two waves per SIMD now overlap).  B8 H12 T2048, the
+  // serial body with operands in LDS -> this: M = 4 148 -> 142 us, M = 2
+  // 123 -> 116, M = 1 114 -> 108, sum M = 4 387 -> 358.  A third ring slot
+  // spills (M = 4 170 us).
   auto tile_pipe = [&](int n) __attribute__((always_inline)) {
     constexpr int NU = SUM ? M * M : M;
     const int buf = n % NB;
