@@ -143,12 +143,25 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """A tensor's address as the C calls' ``void*`` arguments take it."""
+    return None if t is None else t.data_ptr()
 
 
-def stream_of(t: torch.Tensor):
-    """Current HIP stream of the tensor's device, as a void pointer."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# the raw handle of a device's current stream, without building a Stream
+# object for it (2.2 against 0.13 us per call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def stream_of(t: torch.Tensor) -> int:
+    """Current HIP stream of the tensor's device, as an address."""
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def as_dtype(t: torch.Tensor, dt: torch.dtype) -> torch.Tensor:
+    """``t.to(dt)``, without the call where it would return ``t`` itself."""
+    return t if t.dtype is dt else t.to(dt)
 
 
 _scratch_by_stream: dict = {}
@@ -183,7 +196,7 @@ def split_decode_pays(rows: int) -> bool:
 
 def require_device(*ts: torch.Tensor) -> None:
     for t in ts:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(
                 "linatt_amd runs only on a ROCm GPU device; got a tensor on "
                 f"{t.device} (there is no CPU path)")

@@ -85,7 +85,7 @@ class _L2Norm(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         y, rstd = ctx.saved_tensors
-        dy = dy.to(y.dtype).contiguous()
+        dy = _lib.as_dtype(dy, y.dtype).contiguous()
         dx = torch.empty_like(y)
         L = _lib.load()
         n, d = y.numel() // y.shape[-1], y.shape[-1]
@@ -110,8 +110,8 @@ class ChunkDeltaRuleFunction(torch.autograd.Function):
         B, T, H, K = q.shape
         V = v.shape[-1]
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        beta_f = beta.float().contiguous()
-        g_f = g.float().contiguous() if g is not None else None
+        beta_f = _lib.as_dtype(beta, torch.float32).contiguous()
+        g_f = _lib.as_dtype(g, torch.float32).contiguous() if g is not None else None
         h0 = initial_state.float().contiguous() if initial_state is not None else None
         if h0 is not None and h0.shape != (B, H, K, V):
             raise ValueError(f"initial_state must be (B, H, K, V) = {(B, H, K, V)}")
@@ -139,7 +139,7 @@ class ChunkDeltaRuleFunction(torch.autograd.Function):
         V = v.shape[-1]
         dt = _lib.dtype_code(q.dtype)
         L = _lib.load()
-        do = do.to(v.dtype).contiguous()
+        do = _lib.as_dtype(do, v.dtype).contiguous()
         dht = dht.float().contiguous() if dht is not None else None
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         dbeta = torch.empty(B, T, H, device=q.device, dtype=torch.float32)
@@ -153,8 +153,8 @@ class ChunkDeltaRuleFunction(torch.autograd.Function):
             _lib.ptr(dv), _lib.ptr(dbeta), _lib.ptr(dg), _lib.ptr(dh0), B, T, H, K, V,
             float(ctx.scale), dt, _lib.stream_of(q)))
         bdt, gdt, hdt = ctx.dtypes
-        return (dq, dk, dv, dbeta.to(bdt), dg.to(gdt) if dg is not None else None, None,
-                dh0.to(hdt) if dh0 is not None else None, None)
+        return (dq, dk, dv, _lib.as_dtype(dbeta, bdt), _lib.as_dtype(dg, gdt) if dg is not None else None, None,
+                _lib.as_dtype(dh0, hdt) if dh0 is not None else None, None)
 
 
 def _check_kwargs(fn, kwargs):

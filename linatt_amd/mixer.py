@@ -32,6 +32,7 @@ a norm bias) raise.
 
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -308,21 +309,26 @@ class _QKPrologueFn(torch.autograd.Function):
         H, D, W, act, norm, eps, rw, rot, base, offset, inter = ctx.cfg
         B, T, C = x.shape
         L = _lib.load()
-        dy = dy.to(x.dtype).contiguous()
+        dy = _lib.as_dtype(dy, x.dtype).contiguous()
         dx = torch.empty_like(x)
         dw = torch.empty(C, W, device=x.device, dtype=torch.float32)
         db = torch.empty(C, device=x.device, dtype=torch.float32) if b is not None else None
         dnw = torch.empty(D, device=x.device, dtype=torch.float32) if nw is not None else None
-        ws = torch.empty(L.linatt_qk_prologue_bwd_workspace_bytes(B, T, H, D, W),
-                         device=x.device, dtype=torch.uint8)
+        ws = torch.empty(_qk_bwd_workspace_bytes(B, T, H, D, W), device=x.device, dtype=torch.uint8)
         _lib.check("linatt_qk_prologue_bwd", L.linatt_qk_prologue_bwd(
             _lib.ptr(x), _lib.ptr(w2), _lib.ptr(b), _lib.ptr(cache), _lib.ptr(nw), _lib.ptr(dy),
             _lib.ptr(dx), _lib.ptr(dw), _lib.ptr(db), _lib.ptr(dnw), _lib.ptr(ws), B, T, H, D, W,
             act, norm, eps, rw, rot, base, offset, inter, _lib.dtype_code(x.dtype),
             _lib.stream_of(x)))
         wdt, bdt, ndt = ctx.dtypes
-        return (dx, dw.reshape(ctx.wshape).to(wdt), db.to(bdt) if db is not None else None,
-                dnw.to(ndt) if dnw is not None else None, None, None, None)
+        return (dx, _lib.as_dtype(dw.reshape(ctx.wshape), wdt),
+                _lib.as_dtype(db, bdt) if db is not None else None,
+                _lib.as_dtype(dnw, ndt) if dnw is not None else None, None, None, None)
+
+
+@functools.lru_cache(maxsize=256)
+def _qk_bwd_workspace_bytes(*args):
+    return _lib.load().linatt_qk_prologue_bwd_workspace_bytes(*args)
 
 
 def qk_prologue(x, conv_weight, conv_bias=None, *, head_dim, activation="silu", norm="rmsnorm",

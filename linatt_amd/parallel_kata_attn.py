@@ -59,8 +59,8 @@ def _prep(q, k, v):
     (``kata/parallel_kata_attn.py:229-238``)."""
     _lib.require_device(q, k, v)
     dt = v.dtype
-    q = q.to(dt).contiguous()
-    k = k.to(dt).contiguous()
+    q = _lib.as_dtype(q, dt).contiguous()
+    k = _lib.as_dtype(k, dt).contiguous()
     v = v.contiguous()
     B, T, HQ, dk = q.shape
     H = k.shape[2]
@@ -102,23 +102,27 @@ def _fwd_workspace_bytes(*args):
 
 def _bwd(q, k, v, o, den, do, num_groups, scale, variant):
     q, k, v = _prep(q, k, v)
-    do = do.to(v.dtype).contiguous()
+    do = _lib.as_dtype(do, v.dtype).contiguous()
     o = o.contiguous()
-    den = den.float().contiguous()
+    den = _lib.as_dtype(den, torch.float32).contiguous()
     B, T, HQ, dk = q.shape
     H, dv = k.shape[2], v.shape[-1]
     dq = torch.empty_like(q)
     dk_ = torch.empty_like(k)
     dv_ = torch.empty_like(v)
     L = _lib.load()
-    ws = torch.empty(L.linatt_kata_bwd_workspace_bytes(B, T, HQ, dv, _lib.dtype_code(v.dtype)) // 4,
-                     device=q.device, dtype=torch.float32)
+    code = _lib.dtype_code(v.dtype)
+    ws = torch.empty(_bwd_workspace_bytes(B, T, HQ, dv, code) // 4, device=q.device, dtype=torch.float32)
     _lib.check("linatt_kata_bwd", L.linatt_kata_bwd(
         _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(den), _lib.ptr(do),
         _lib.ptr(dq), _lib.ptr(dk_), _lib.ptr(dv_), _lib.ptr(ws),
-        B, T, HQ, H, dk, dv, num_groups, float(scale), _VARIANT[variant],
-        _lib.dtype_code(v.dtype), _lib.stream_of(q)))
+        B, T, HQ, H, dk, dv, num_groups, float(scale), _VARIANT[variant], code, _lib.stream_of(q)))
     return dq, dk_, dv_
+
+
+@functools.lru_cache(maxsize=256)
+def _bwd_workspace_bytes(*args):
+    return _lib.load().linatt_kata_bwd_workspace_bytes(*args)
 
 
 def parallel_kata_attn_fwd_impl(q, k, v, num_groups, scale, bT, bK, c=None):
@@ -166,7 +170,8 @@ class ParallelKataAttnFunction(torch.autograd.Function):
         q, k, v, o, den = ctx.saved_tensors
         dq, dk, dv = parallel_kata_attn_bwd(q, k, v, o, den, do, ctx.num_groups, ctx.scale)
         qd, kd, vd = ctx.dtypes
-        return dq.to(qd), dk.to(kd), dv.to(vd), None, None, None, None, None
+        return (_lib.as_dtype(dq, qd), _lib.as_dtype(dk, kd), _lib.as_dtype(dv, vd), None, None, None, None,
+                None)
 
 
 def parallel_kata_attn(q, k, v, num_groups=4, scale=None, bT=64, bK=64, use_triton_bwd=True):
@@ -214,7 +219,8 @@ class ParallelKataAttnSumFunction(torch.autograd.Function):
         q, k, v, o, den = ctx.saved_tensors
         dq, dk, dv = parallel_kata_attn_bwd_sum(q, k, v, o, den, do, ctx.num_groups, ctx.scale)
         qd, kd, vd = ctx.dtypes
-        return dq.to(qd), dk.to(kd), dv.to(vd), None, None, None, None, None
+        return (_lib.as_dtype(dq, qd), _lib.as_dtype(dk, kd), _lib.as_dtype(dv, vd), None, None, None, None,
+                None)
 
 
 def parallel_kata_attn_sum(q, k, v, num_groups=4, scale=None, bT=64, bK=64, use_triton_bwd=True):
@@ -248,7 +254,7 @@ class _KataDecayFunction(torch.autograd.Function):
         q, k, v, c, o, den = ctx.saved_tensors
         qc, kc, vc = _prep(q, k, v)
         cf = c.float().contiguous()
-        do = do.to(vc.dtype).contiguous()
+        do = _lib.as_dtype(do, vc.dtype).contiguous()
         B, T, HQ, dk = qc.shape
         H, dv = kc.shape[2], vc.shape[-1]
         dq, dk_, dv_ = torch.empty_like(qc), torch.empty_like(kc), torch.empty_like(vc)
@@ -258,7 +264,7 @@ class _KataDecayFunction(torch.autograd.Function):
         oc = o.contiguous()
         denc = den.float().contiguous()
         L = _lib.load()
-        ws = torch.empty(L.linatt_kata_bwd_workspace_bytes(B, T, HQ, dv, _lib.dtype_code(vc.dtype)) // 4,
+        ws = torch.empty(_bwd_workspace_bytes(B, T, HQ, dv, _lib.dtype_code(vc.dtype)) // 4,
                          device=q.device, dtype=torch.float32)
         _lib.check("linatt_kata_bwd_decay", L.linatt_kata_bwd_decay(
             _lib.ptr(qc), _lib.ptr(kc), _lib.ptr(vc), _lib.ptr(cf), _lib.ptr(oc),
@@ -266,7 +272,8 @@ class _KataDecayFunction(torch.autograd.Function):
             _lib.ptr(dv_), _lib.ptr(dc), _lib.ptr(ws), B, T, HQ, H, dk, dv, ctx.num_groups,
             float(ctx.scale), _lib.dtype_code(vc.dtype), _lib.stream_of(qc)))
         qd, kd, vd, cd = ctx.dtypes
-        return dq.to(qd), dk_.to(kd), dv_.to(vd), dc.to(cd), None, None
+        return (_lib.as_dtype(dq, qd), _lib.as_dtype(dk_, kd), _lib.as_dtype(dv_, vd), _lib.as_dtype(dc, cd),
+                None, None)
 
 
 def parallel_kata_attn_decay(q, k, v, c, num_groups=2, scale=None):
@@ -331,7 +338,7 @@ class _KataONormFunction(torch.autograd.Function):
         num_groups, scale, variant = ctx.args
         B, T, HQ, dk = q.shape
         H, dv = k.shape[2], v.shape[-1]
-        dy = dy.to(v.dtype).contiguous()
+        dy = _lib.as_dtype(dy, v.dtype).contiguous()
         dq, dk_, dv_ = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         dc = torch.empty_like(cf) if cf is not None else None
         dw = torch.empty(dv, device=q.device, dtype=torch.float32) if w is not None else None
@@ -344,8 +351,9 @@ class _KataONormFunction(torch.autograd.Function):
             _lib.ptr(dc), _lib.ptr(dw), _lib.ptr(ws), B, T, HQ, H, dk, dv, num_groups, scale,
             _VARIANT[variant], _lib.dtype_code(v.dtype), _lib.stream_of(q)))
         qd, kd, vd, cd, wd = ctx.dtypes
-        return (dq.to(qd), dk_.to(kd), dv_.to(vd), dc.to(cd) if dc is not None else None,
-                dw.to(wd) if dw is not None else None, None, None, None, None)
+        return (_lib.as_dtype(dq, qd), _lib.as_dtype(dk_, kd), _lib.as_dtype(dv_, vd),
+                _lib.as_dtype(dc, cd) if dc is not None else None,
+                _lib.as_dtype(dw, wd) if dw is not None else None, None, None, None, None)
 
 
 def parallel_kata_attn_onorm(q, k, v, norm_weight=None, eps=1e-5, num_groups=4, scale=None,
