@@ -93,6 +93,20 @@ int linatt_kata_bwd(const void* q, const void* k, const void* v, const void* o,
                     void* workspace, int B, int T, int HQ, int H, int dk_dim, int dv_dim,
                     int num_groups, float scale, int variant, int dtype, void* stream);
 
+/* linatt_kata_bwd with the dk/dv pass's query tiles split over more workgroups
+ * where it leaves CUs idle (bfloat16, dk = 64: few kv heads, or grouped
+ * queries), its float32 partial sums in the workspace behind the backward's
+ * own and added in order by a third launch.  workspace:
+ * linatt_kata_bwd_split_workspace_bytes bytes, 16-byte aligned.  Same results
+ * as linatt_kata_bwd up to the float32 summation order. */
+size_t linatt_kata_bwd_split_workspace_bytes(int B, int T, int HQ, int H, int dk, int dv,
+                                             int num_groups, int variant, int dtype);
+int linatt_kata_bwd_split(const void* q, const void* k, const void* v, const void* o,
+                          const float* den, const void* dout, void* dq, void* dk, void* dv,
+                          void* workspace, size_t workspace_bytes, int B, int T, int HQ, int H,
+                          int dk_dim, int dv_dim, int num_groups, float scale, int variant,
+                          int dtype, void* stream);
+
 /* Backward of the decayed concat score A[t,s] * exp(min(c_t - c_s, 0)):
  * dq, dk, dv as linatt_kata_bwd plus dc (B,T,HQ) float32, the gradient of the
  * cumulative log-decay c.  Replaces the O(T^2)-memory autograd recompute of

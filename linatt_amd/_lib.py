@@ -42,6 +42,8 @@ SIGNATURES = {
     "linatt_kata_fwd_split": (_i, [_vp] * 7 + [_sz] + [_i] * 7 + [_f, _i, _i, _vp]),
     "linatt_kata_bwd_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "linatt_kata_bwd": (_i, [_vp] * 10 + [_i] * 7 + [_f, _i, _i, _vp]),
+    "linatt_kata_bwd_split_workspace_bytes": (_sz, [_i] * 9),
+    "linatt_kata_bwd_split": (_i, [_vp] * 10 + [_sz] + [_i] * 7 + [_f, _i, _i, _vp]),
     "linatt_kata_bwd_dq": (_i, [_vp] * 10 + [_i] * 7 + [_f, _i, _i, _vp]),
     "linatt_kata_bwd_decay": (_i, [_vp] * 12 + [_i] * 7 + [_f, _i, _vp]),
     "linatt_kata_bwd_dkdv": (_i, [_vp] * 10 + [_i] * 7 + [_f, _i, _i, _vp]),

@@ -283,6 +283,20 @@ size_t linatt_kata_bwd_workspace_bytes(int B, int T, int HQ, int dv_dim, int dty
   return linatt::kata_dop_offset(rows) + dop;
 }
 
+// tiles per workgroup of a split dk/dv pass (0: unsplit), and its workspace:
+// the backward's, then the partial blocks
+static int bwd_split(int B, int T, int HQ, int H, int dk, int dv, int M, int variant, int dtype) {
+  if (dtype != LINATT_BFLOAT16 || dk != 64 || !compiled(dtype, dk, dv, M)) return 0;
+  return kata_dkdv_split((int64_t)B * H, T, HQ / H, kata_dkdv_tile_time(M, variant == LINATT_KATA_SUM));
+}
+static size_t bwd_part_offset(int B, int T, int HQ, int dv, int dtype) {
+  return (linatt_kata_bwd_workspace_bytes(B, T, HQ, dv, dtype) + 255) & ~size_t(255);
+}
+static size_t bwd_split_ws(int B, int T, int HQ, int H, int dv, int L, int dtype) {
+  const size_t off = bwd_part_offset(B, T, HQ, dv, dtype);
+  return L ? off + kata_dkdv_part_bytes((int64_t)B * H, T, HQ / H, L) : off;
+}
+
 // Shared body of the three backward entry points; `parts` selects the
 // kernels (KATA_BWD_DQ and/or KATA_BWD_DKDV).  Pointers a part does not use
 // may be null.
@@ -290,7 +304,8 @@ static int kata_bwd_entry(const char* fn, int parts, const void* q, const void* 
                           const void* o, const float* den, const void* dout, void* dq, void* dk,
                           void* dv, void* workspace, int B, int T, int HQ, int H, int dk_dim,
                           int dv_dim, int num_groups, float scale, int variant, int dtype,
-                          void* stream, const float* c = nullptr, float* dc = nullptr) {
+                          void* stream, const float* c = nullptr, float* dc = nullptr,
+                          bool split = false, size_t ws_bytes = 0) {
   g_last_error.clear();
   int st = check_common(B, T, HQ, H, dk_dim, dv_dim, num_groups, scale, variant, dtype);
   if (st) return st;
@@ -309,6 +324,14 @@ static int kata_bwd_entry(const char* fn, int parts, const void* q, const void* 
   a.scale = scale;
   a.c = c;
   a.dc = dc;
+  if (split) {
+    a.split = bwd_split(B, T, HQ, H, dk_dim, dv_dim, num_groups, variant, dtype);
+    if (a.split) {
+      if (ws_bytes < bwd_split_ws(B, T, HQ, H, dv_dim, a.split, dtype))
+        return fail(LINATT_EINVAL, std::string(fn) + ": workspace smaller than linatt_kata_bwd_split_workspace_bytes");
+      a.part = (float*)((char*)workspace + bwd_part_offset(B, T, HQ, dv_dim, dtype));
+    }
+  }
   bool found = false;
   hipError_t e = dispatch_bwd(a, parts, dtype, variant, c != nullptr, (hipStream_t)stream, &found);
   if (!found)
@@ -326,6 +349,22 @@ int linatt_kata_bwd(const void* q, const void* k, const void* v, const void* o,
   return kata_bwd_entry("linatt_kata_bwd", KATA_BWD_DQ | KATA_BWD_DKDV, q, k, v, o, den, dout,
                         dq, dk, dv, workspace, B, T, HQ, H, dk_dim, dv_dim, num_groups, scale,
                         variant, dtype, stream);
+}
+
+size_t linatt_kata_bwd_split_workspace_bytes(int B, int T, int HQ, int H, int dk_dim, int dv_dim,
+                                             int num_groups, int variant, int dtype) {
+  if (check_common(B, T, HQ, H, dk_dim, dv_dim, num_groups, 1.f, variant, dtype)) return 0;
+  return bwd_split_ws(B, T, HQ, H, dv_dim, bwd_split(B, T, HQ, H, dk_dim, dv_dim, num_groups, variant, dtype), dtype);
+}
+
+int linatt_kata_bwd_split(const void* q, const void* k, const void* v, const void* o,
+                          const float* den, const void* dout, void* dq, void* dk, void* dv,
+                          void* workspace, size_t workspace_bytes, int B, int T, int HQ, int H,
+                          int dk_dim, int dv_dim, int num_groups, float scale, int variant, int dtype,
+                          void* stream) {
+  return kata_bwd_entry("linatt_kata_bwd_split", KATA_BWD_DQ | KATA_BWD_DKDV, q, k, v, o, den, dout, dq, dk, dv,
+                        workspace, B, T, HQ, H, dk_dim, dv_dim, num_groups, scale, variant, dtype, stream, nullptr,
+                        nullptr, true, workspace_bytes);
 }
 
 int linatt_kata_bwd_decay(const void* q, const void* k, const void* v, const float* c,

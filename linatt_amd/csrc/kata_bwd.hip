@@ -22,6 +22,7 @@
 // of 64 stream through LDS as Q, Q^T, dO, dO^T plus delta and 1/D.
 #include "common.h"
 #include "kata_kernels.h"
+#include "kata_split.h"
 
 namespace linatt {
 
@@ -772,12 +773,14 @@ __global__ __launch_bounds__(256, 2) void kata_bwd_dq_tile_kernel(
 template <int DK>
 constexpr int kata_dkdv_waves() { return DK == 64 ? 4 : 8; }
 
-template <typename T, int DK, int DV, int M, bool SUM, bool DECAY>
+// SPLIT: the workgroup's run of a split launch (kata_split.h), whose sums go to
+// partial blocks where the list was cut
+template <typename T, int DK, int DV, int M, bool SUM, bool DECAY, bool SPLIT>
 __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_tile_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
     const float* __restrict__ den, const float* __restrict__ delta, const T* __restrict__ dout,
     T* __restrict__ dk, T* __restrict__ dv, const float* __restrict__ c, float* __restrict__ dc,
-    int Tn, int HQ, int H, float scale2, int nst, int nbh) {
+    int Tn, int HQ, int H, float scale2, int nst, int nbh, int split, float* __restrict__ part) {
   constexpr int E = DK / M;
   constexpr int KE = E / 16;
   constexpr float kPScale = __is_same(T, _Float16) ? 4096.f : 1.f;
@@ -805,7 +808,15 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
   const int cl = lane & 31, hh = lane >> 5;
   int stile, bh;
-  map_block(blockIdx.x, nst, nbh, stile, bh, false);
+  SplitRun run{};
+  if constexpr (SPLIT) {
+    int item;
+    map_block(blockIdx.x, gridDim.x / nbh, nbh, item, bh, false);
+    run = kata_dkdv_run(item, Tn, HQ / H, split);
+    stile = run.tile;
+  } else {
+    map_block(blockIdx.x, nst, nbh, stile, bh, false);
+  }
   const int b = bh / H, h = bh % H;
   const int G = HQ / H;
   const int s0 = stile * 32 * NW;
@@ -858,7 +869,8 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
 
   // query tiles (hq, tt) of this key tile, flattened over the G query heads
   const int ntt = (Tn + 63) / 64, tt0 = s0 / 64, nq = ntt - tt0;
-  const int ntiles = G * nq;
+  // flattened tiles [n0, ntiles) of this workgroup
+  const int n0 = SPLIT ? run.lo : 0, ntiles = SPLIT ? run.hi : G * nq;
   // tile n: copies CPW w .. CPW w + CPW - 1 of each sub-tile of q and of dO by
   // wave w (full tiles from a scalar base plus these per-lane offsets; a
   // head's last tile clamps rows)
@@ -911,8 +923,8 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
 
   float csl = (DECAY && svalid) ? c[((int64_t)b * Tn + sl) * HQ + h * G] : 0.f;
   vm_drain();  // k, v (and c) of this wave's keys are in registers
-  issue(0, 0);
-  load_rows(0, 0);
+  issue(n0, n0 % NB);
+  load_rows(n0, n0 % NB);
   float dcc = 0.f;
   // query tile n (global index over the G heads) with or without the causal /
   // past-T masks: only the NW / 2 tiles on this workgroup's diagonal and a
@@ -1192,14 +1204,37 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
   const int nfull = Tn / 64 - tt0;
   for (int hi = 0; hi < G; ++hi) {
     const int nb = hi * nq;
-    int i = 0;
-    for (; i < nq && i < NW / 2; ++i) tile(nb + i, BoolC<true>{});
+    int i = SPLIT ? max(0, n0 - nb) : 0;
+    const int nq_e = SPLIT ? min(nq, ntiles - nb) : nq, nfull_e = SPLIT ? min(nfull, nq_e) : nfull;
+    for (; i < nq_e && i < NW / 2; ++i) tile(nb + i, BoolC<true>{});
     if constexpr (kPipe) {
-      for (; i < nfull; ++i) tile_pipe(nb + i);
+      for (; i < nfull_e; ++i) tile_pipe(nb + i);
     } else {
-      for (; i < nfull; ++i) tile(nb + i, BoolC<false>{});
+      for (; i < nfull_e; ++i) tile(nb + i, BoolC<false>{});
     }
-    for (; i < nq; ++i) tile(nb + i, BoolC<true>{});
+    for (; i < nq_e; ++i) tile(nb + i, BoolC<true>{});
+  }
+
+  if constexpr (SPLIT) {
+    static_assert(kPipe, "bf16, dk = 64, no decay");
+    if (run.pieces > 1) {
+      float* p = part + dkdv_part_offset(run.piece, nbh, bh, nst, 4 * stile + w) + 4 * lane;
+#pragma unroll
+      for (int db = 0; db < DV / 32; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *reinterpret_cast<f32x4*>(p + 256 * (4 * db + i)) =
+              f32x4{dva[db][4 * i], dva[db][4 * i + 1], dva[db][4 * i + 2], dva[db][4 * i + 3]};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        f32x4 y;
+        if constexpr (k16) y = dk16[e >> 1][e & 1];
+        else y = f32x4{dka[e >> 2][4 * (e & 3)], dka[e >> 2][4 * (e & 3) + 1], dka[e >> 2][4 * (e & 3) + 2],
+                       dka[e >> 2][4 * (e & 3) + 3]};
+        *reinterpret_cast<f32x4*>(p + 256 * (8 + e)) = y;
+      }
+      return;
+    }
   }
 
   if constexpr (k16) {
@@ -1236,6 +1271,35 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
         st4<T>(dvrow + 32 * db + 8 * i + 4 * hh,
                to4<T>(dva[db][4 * i] * kPInv, dva[db][4 * i + 1] * kPInv,
                       dva[db][4 * i + 2] * kPInv, dva[db][4 * i + 3] * kPInv));
+  }
+}
+
+// The split dk/dv pass's outputs where the list was cut: a wave per 32 keys,
+// the pieces added in order, stored as the unsplit kernel stores its registers.
+template <typename T, bool K16>
+__global__ __launch_bounds__(256) void kata_dkdv_split_finish_kernel(const float* __restrict__ part, T* __restrict__ dk,
+                                                                     T* __restrict__ dv, int Tn, int H, int G, int nkt,
+                                                                     int nbk, int split) {
+  const int lane = threadIdx.x & 63, cl = lane & 31, hh = lane >> 5, w = wave_id();
+  const int st = blockIdx.x % nkt, bh = blockIdx.x / nkt;
+  const int pieces = split_pieces(kata_query_tiles(st, Tn, G), split);
+  if (pieces == 1) return;
+  f32x4 x[16] = {};
+  for (int i = 0; i < pieces; ++i) {
+    const float* p = part + dkdv_part_offset(i, nbk, bh, nkt, 4 * st + w) + 4 * lane;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) x[e] += *reinterpret_cast<const f32x4*>(p + 256 * e);
+  }
+  const int sw = 128 * st + 32 * w;
+  const int64_t row0 = (int64_t)(bh / H) * Tn * H + bh % H;
+  auto out = [&](T* base, int s, int d, const f32x4& y, float f) __attribute__((always_inline)) {
+    if (s < Tn) st4<T>(base + (row0 + (int64_t)s * H) * 64 + d, to4<T>(y[0] * f, y[1] * f, y[2] * f, y[3] * f));
+  };
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    out(dv, sw + cl, 8 * e + 4 * hh, x[e], 1.f);
+    if constexpr (K16) out(dk, sw + 16 * (e & 1) + (lane & 15), 16 * (e >> 1) + 4 * (lane >> 4), x[8 + e], 2.f);
+    else out(dk, sw + cl, 8 * e + 4 * hh, x[8 + e], 2.f);
   }
 }
 
@@ -1280,9 +1344,22 @@ hipError_t launch_kata_bwd(const KataArgs& a, int parts, hipStream_t stream) {
       if constexpr (kTiles) {
         constexpr int kw = kata_dkdv_waves<DK>();
         const int nkt = (a.T + 32 * kw - 1) / (32 * kw);
-        kata_bwd_dkdv_tile_kernel<T, DK, DV, M, SUM, DECAY><<<dim3(nkt * nbk), dim3(64 * kw), 0, stream>>>(
-            (const T*)a.q, (const T*)a.k, (const T*)a.v, a.den, a.delta, (const T*)a.dout,
-            (T*)a.dk, (T*)a.dv, a.c, a.dc, a.T, a.HQ, a.H, scale2, nkt, nbk);
+        auto go = [&](auto sp, int wgs) {
+          kata_bwd_dkdv_tile_kernel<T, DK, DV, M, SUM, DECAY, decltype(sp)::value>
+              <<<dim3(wgs), dim3(64 * kw), 0, stream>>>(
+                  (const T*)a.q, (const T*)a.k, (const T*)a.v, a.den, a.delta, (const T*)a.dout,
+                  (T*)a.dk, (T*)a.dv, a.c, a.dc, a.T, a.HQ, a.H, scale2, nkt, nbk, a.split, a.part);
+        };
+        if (!a.split) {
+          go(BoolC<false>{}, nkt * nbk);
+        } else if constexpr (__is_same(T, __bf16) && DK == 64 && !DECAY) {
+          const int G = a.HQ / a.H;
+          go(BoolC<true>{}, kata_dkdv_items(a.T, G, a.split) * nbk);
+          kata_dkdv_split_finish_kernel<T, DK / M == 16><<<dim3(nkt * nbk), dim3(256), 0, stream>>>(
+              a.part, (T*)a.dk, (T*)a.dv, a.T, a.H, G, nkt, nbk, a.split);
+        } else {
+          return hipErrorInvalidValue;
+        }
       } else
       kata_bwd_dkdv_kernel<T, DK, DV, M, SUM, DECAY><<<dim3(nqt * nbk), dim3(256), 0, stream>>>(
           (const T*)a.q, (const T*)a.k, (const T*)a.v, a.den, a.delta, (const T*)a.dout,

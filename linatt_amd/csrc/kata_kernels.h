@@ -41,8 +41,9 @@ struct KataArgs {
   // numerator num = o den = sum_s A[t,s] v_s is written here in float32
   // instead of o (o may then be null)
   float* num32;
-  // forward: tiles per workgroup of a split launch (kata_split.h; 0: unsplit)
-  // and its partial blocks (pieces, B HQ, 4 ceil(T / 128), kFwdPart) float32
+  // tiles per workgroup of a split launch (kata_split.h; 0: unsplit) and its
+  // float32 partial blocks: forward (pieces, B HQ, 4 ceil(T / 128), kFwdPart),
+  // dk/dv pass (pieces, B H, 4 ceil(T / 128), kDkdvPart)
   int split;
   float* part;
 };

@@ -55,18 +55,19 @@ constexpr int kFwdPart = 32 * 64 + 64;
 constexpr int kMaxPieces = 16;
 
 // A workgroup's time per tile alone on its CU and with the CU full (slots / 256
-// workgroups sharing it).
+// workgroups sharing it), and what a split adds to the call.
 struct TileTime {
   double solo_us, full_us;
   int slots;
+  double split_us;
 };
 
 // Tiles per workgroup with the least modelled time, 0 to leave the launch
 // unsplit.  Modelled as the longer of the longest list at the solo rate and
 // the whole work over all slots at the full rate; for a split the rate of its
-// runs is 1.3 solo and half a run is left uneven at the end, and it adds 8 us
-// (the second launch, and the first tile's latency in every workgroup) and the
-// partial blocks written and read at 4.5 TB/s.  It has to win by a tenth.
+// runs is 1.3 solo and half a run is left uneven at the end, and it adds
+// split_us (the second launch, and the first tile's latency in every workgroup)
+// and the partial blocks written and read at 4.5 TB/s.  It has to win by a tenth.
 template <typename Lists>
 inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileTime& tt, double list_bytes) {
   int64_t units = 0;
@@ -87,7 +88,7 @@ inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileT
       const int p = split_pieces(lists(i), L);
       if (p > 1) part += p;
     }
-    const double t = longer(1.3 * L * tt.solo_us, all + 0.5 * L * tt.solo_us) + 8. +
+    const double t = longer(1.3 * L * tt.solo_us, all + 0.5 * L * tt.solo_us) + tt.split_us +
                      (double)(part * heads) * list_bytes * (2. / 4.5e6);
     if (t < best) {
       best = t;
@@ -105,12 +106,12 @@ inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileT
 // concat M = 4 28 -> 26.  Left unsplit: concat M = 4 at B2 T2048 (30 against 33),
 // B4 (39 against 51), M = 1 at B1 T1500 (18 against 19).
 inline TileTime kata_fwd_tile_time(int elt_bytes, bool fp16, int dk, int M, bool sum, bool decay) {
-  if (elt_bytes == 4) return {6., 14., 512};
+  if (elt_bytes == 4) return {6., 14., 512, 8.};
   double solo = sum && M > 1 ? (M == 2 ? 1.3 : 2.4) : 0.85;
   if (dk == 128) solo *= 1.4;
   if (decay) solo *= 1.4;
   if (fp16) solo *= 1.4;
-  return dk == 128 ? TileTime{solo, 1.4 * solo, 512} : TileTime{solo, 2.2 * solo, 768};
+  return dk == 128 ? TileTime{solo, 1.4 * solo, 512, 8.} : TileTime{solo, 2.2 * solo, 768, 8.};
 }
 inline int kata_fwd_split(int64_t BH, int T, const TileTime& tt) {
   return best_split([&](int qt) { return kata_key_tiles(qt, T); }, BH, (T + 127) / 128, tt, 4. * kFwdPart * 4);
@@ -119,6 +120,54 @@ inline int kata_fwd_split(int64_t BH, int T, const TileTime& tt) {
 inline size_t kata_fwd_part_bytes(int64_t BH, int T, int L) {
   const int nqt = (T + 127) / 128;
   return (size_t)split_pieces(kata_key_tiles(nqt - 1, T), L) * BH * 4 * nqt * kFwdPart * sizeof(float);
+}
+
+// dk/dv (bf16, dk = 64, no decay): the list of key tile st (128 keys) is the
+// query tiles of 64 at or after it, over the G query heads of its kv head.
+__host__ __device__ inline int kata_query_tiles(int st, int T, int G) { return G * ((T + 63) / 64 - 2 * st); }
+inline int kata_dkdv_items(int T, int G, int L) {
+  int n = 0;
+  for (int st = 0; st < (T + 127) / 128; ++st) n += split_pieces(kata_query_tiles(st, T, G), L);
+  return n;
+}
+// item j of a kv head, longest lists (first key tiles) first
+__device__ __forceinline__ SplitRun kata_dkdv_run(int j, int T, int G, int L) {
+  SplitRun r;
+  r.tile = 0;
+  int n = kata_query_tiles(0, T, G);
+  r.pieces = split_pieces(n, L);
+  while (j >= r.pieces) {
+    j -= r.pieces;
+    ++r.tile;
+    n = kata_query_tiles(r.tile, T, G);
+    r.pieces = split_pieces(n, L);
+  }
+  r.piece = j;
+  const int per = (n + r.pieces - 1) / r.pieces;
+  r.lo = j * per;
+  r.hi = r.lo + per < n ? r.lo + per : n;
+  return r;
+}
+// floats of a wave's partial block: 32 keys x (64 dk + 64 dv)
+constexpr int kDkdvPart = 32 * 128;
+__host__ __device__ inline int64_t dkdv_part_offset(int piece, int nbk, int bh, int nkt, int blk) {
+  return (((int64_t)piece * nbk + bh) * (4 * nkt) + blk) * kDkdvPart;
+}
+// Per 64-query tile of 128 keys, two workgroups per CU.  Unsplit -> split, us:
+// sum M = 2 B6 T1403 HQ12 H4 124 -> 105; concat M = 4 B1 H12 T2048 59 -> 47, B2
+// HQ16 H8 T2048 112 -> 86; M = 1 B1 HQ8 H4 T3000 108 -> 55; sum M = 4 B1 H12
+// T2048 141 -> 90.  Left unsplit: M = 1 B1 H8 T1500 (33 against 35), concat M = 4
+// B1 H4 T1000 (33 against 34).
+inline TileTime kata_dkdv_tile_time(int M, bool sum) {
+  const double full = sum && M > 1 ? (M == 2 ? 3.2 : 7.0) : M == 1 ? 2.1 : M == 2 ? 2.3 : 2.8;
+  return {full / 1.6, full, 512, 13.};
+}
+inline int kata_dkdv_split(int64_t BH, int T, int G, const TileTime& tt) {
+  return best_split([&](int st) { return kata_query_tiles(st, T, G); }, BH, (T + 127) / 128, tt, 4. * kDkdvPart * 4);
+}
+inline size_t kata_dkdv_part_bytes(int64_t BH, int T, int G, int L) {
+  const int nkt = (T + 127) / 128;
+  return (size_t)split_pieces(kata_query_tiles(0, T, G), L) * BH * 4 * nkt * kDkdvPart * sizeof(float);
 }
 
 }  // namespace linatt

@@ -111,13 +111,19 @@ def _bwd(q, k, v, o, den, do, num_groups, scale, variant):
     dk_ = torch.empty_like(k)
     dv_ = torch.empty_like(v)
     L = _lib.load()
-    code = _lib.dtype_code(v.dtype)
-    ws = torch.empty(_bwd_workspace_bytes(B, T, HQ, dv, code) // 4, device=q.device, dtype=torch.float32)
-    _lib.check("linatt_kata_bwd", L.linatt_kata_bwd(
+    shape, code, var = (B, T, HQ, H, dk, dv, num_groups), _lib.dtype_code(v.dtype), _VARIANT[variant]
+    nws = _bwd_split_workspace_bytes(*shape, var, code)
+    ws = torch.empty(nws, device=q.device, dtype=torch.uint8)
+    _lib.check("linatt_kata_bwd_split", L.linatt_kata_bwd_split(
         _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(den), _lib.ptr(do),
-        _lib.ptr(dq), _lib.ptr(dk_), _lib.ptr(dv_), _lib.ptr(ws),
-        B, T, HQ, H, dk, dv, num_groups, float(scale), _VARIANT[variant], code, _lib.stream_of(q)))
+        _lib.ptr(dq), _lib.ptr(dk_), _lib.ptr(dv_), _lib.ptr(ws), nws, *shape, float(scale), var, code,
+        _lib.stream_of(q)))
     return dq, dk_, dv_
+
+
+@functools.lru_cache(maxsize=256)
+def _bwd_split_workspace_bytes(*args):
+    return _lib.load().linatt_kata_bwd_split_workspace_bytes(*args)
 
 
 @functools.lru_cache(maxsize=256)

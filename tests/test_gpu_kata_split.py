@@ -67,3 +67,44 @@ def test_split_forward_workspace_checked():
     tail = (*shape, 0.25, 0, 0, _lib.stream_of(x))
     for w, n in ((None, 0), (ws, nws - 1), (ws[4:], nws)):
         assert L.linatt_kata_fwd_split(p(x), p(x), p(x), None, p(x), p(den), p(w), n, *tail) == -1
+
+
+@pytest.mark.parametrize("B,T,HQ,H,M,variant", [(6, 1403, 12, 4, 2, "sum"), (1, 2048, 3, 3, 4, "concat"),
+                                                (1, 2100, 4, 1, 4, "concat"), (1, 1985, 6, 2, 1, "concat"),
+                                                (1, 1930, 2, 1, 4, "sum"), (2, 2048, 16, 8, 4, "concat")])
+def test_split_backward_equals_unsplit(B, T, HQ, H, M, variant):
+    """``linatt_kata_bwd_split`` (dk/dv's query tiles over several workgroups)
+    against ``linatt_kata_bwd``: dq is the same kernel (bit for bit); dk, dv
+    add the same products in another order, in float32 far below the bf16
+    spacing they are then rounded to, so a value moves by one spacing (2^-7 of
+    it) at most, and the whole by less than that in the 2-norm."""
+    from linatt_amd import _lib
+    print(f"\nsplit backward B{B} T{T} HQ{HQ} H{H} M{M} {variant}", flush=True)
+    L, p = _lib.load(), _lib.ptr
+    g = torch.Generator().manual_seed(T + M)
+    q, do = (torch.randn(B, T, HQ, 64, generator=g).bfloat16().cuda() for _ in range(2))
+    k, v = (torch.randn(B, T, H, 64, generator=g).bfloat16().cuda() for _ in range(2))
+    o, den = torch.empty_like(q), torch.empty(B, T, HQ, device="cuda")
+    var, sp, sc, shape = int(variant == "sum"), _lib.stream_of(q), math.sqrt(M) / 8, (B, T, HQ, H, 64, 64, M)
+    _lib.check("fwd", L.linatt_kata_fwd(p(q), p(k), p(v), None, p(o), p(den), *shape, sc, var, 1, sp))
+    nb = L.linatt_kata_bwd_workspace_bytes(B, T, HQ, 64, 1)
+    ns = L.linatt_kata_bwd_split_workspace_bytes(*shape, var, 1)
+    assert ns > nb + 256  # the split engages
+    ws = torch.empty(ns, device="cuda", dtype=torch.uint8)
+    out = []
+    for split in (False, True):
+        gr = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+        head, tail = (p(q), p(k), p(v), p(o), p(den), p(do), *map(p, gr), p(ws)), (*shape, sc, var, 1, sp)
+        if split:
+            _lib.check("split", L.linatt_kata_bwd_split(*head, ns, *tail))
+        else:
+            _lib.check("bwd", L.linatt_kata_bwd(*head, *tail))
+        out.append(gr)
+    assert L.linatt_kata_bwd_split(*head, ns - 1, *tail) == -1
+    torch.cuda.synchronize()
+    assert torch.equal(out[0][0], out[1][0])
+    for a, b in zip(out[0][1:], out[1][1:]):
+        a, b = a.double(), b.double()
+        print("  rel %.1e" % ((a - b).norm() / a.norm()).item(), flush=True)
+        assert (a - b).norm() <= 2.0 ** -8 * a.norm()
+        assert ((a - b).abs() <= 2.0 ** -7 * a.abs() + 2.0 ** -12 * a.abs().max()).all()
