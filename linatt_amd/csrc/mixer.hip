@@ -261,39 +261,57 @@ __global__ __launch_bounds__(64) void short_conv_bwd_kernel(ConvArgs a) {
 // ... of the range, eight loads in flight), then one thread per column adds
 // the 32 phase sums.  With split_w > 0 the columns are [c][0 .. split_w - 1
 // weight, split_w bias] of a convolution and go to dw[c][w] and db[c] instead.
+struct ColSum {
+  const float* part;
+  float* out;
+  int np, n, rows_per, split_w;
+  float* db;
+};
+__device__ __forceinline__ void colsum_block(const ColSum& a, int bx, int by, float (&red)[32][33]) {
+  const int c = bx * 32 + (threadIdx.x & 31), k = threadIdx.x >> 5;
+  const int p0 = by * a.rows_per, p1 = min(a.np, p0 + a.rows_per);
+  float s = 0.f;
+  if (c < a.n) {
+    int p = p0 + k;
+    for (; p + 7 * 32 < p1; p += 8 * 32) {
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = a.part[(int64_t)(p + 32 * j) * a.n + c];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += v[j];
+    }
+    for (; p < p1; p += 32) s += a.part[(int64_t)p * a.n + c];
+  }
+  red[k][threadIdx.x & 31] = s;
+  __syncthreads();
+  if (threadIdx.x < 32 && c < a.n) {
+    float t = 0.f;
+#pragma unroll
+    for (int j = 0; j < 32; ++j) t += red[j][threadIdx.x];
+    if (a.split_w == 0) {
+      a.out[(int64_t)by * a.n + c] = t;
+    } else {
+      const int cc = c / (a.split_w + 1), w = c % (a.split_w + 1);
+      if (w < a.split_w) a.out[cc * a.split_w + w] = t;
+      else if (a.db) a.db[cc] = t;
+    }
+  }
+}
 __global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ part,
                                                       float* __restrict__ out, int np, int n,
                                                       int rows_per, int split_w = 0,
                                                       float* __restrict__ db = nullptr) {
   __shared__ float red[32][33];
-  const int c = blockIdx.x * 32 + (threadIdx.x & 31), k = threadIdx.x >> 5;
-  const int p0 = blockIdx.y * rows_per, p1 = min(np, p0 + rows_per);
-  float s = 0.f;
-  if (c < n) {
-    int p = p0 + k;
-    for (; p + 7 * 32 < p1; p += 8 * 32) {
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = part[(int64_t)(p + 32 * j) * n + c];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) s += v[j];
-    }
-    for (; p < p1; p += 32) s += part[(int64_t)p * n + c];
-  }
-  red[k][threadIdx.x & 31] = s;
-  __syncthreads();
-  if (threadIdx.x < 32 && c < n) {
-    float t = 0.f;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) t += red[j][threadIdx.x];
-    if (split_w == 0) {
-      out[(int64_t)blockIdx.y * n + c] = t;
-    } else {
-      const int cc = c / (split_w + 1), w = c % (split_w + 1);
-      if (w < split_w) out[cc * split_w + w] = t;
-      else if (db) db[cc] = t;
-    }
-  }
+  colsum_block(ColSum{part, out, np, n, rows_per, split_w, db}, blockIdx.x, blockIdx.y, red);
+}
+// two sums in one launch: blocks [0, na) of a, the rest of b.  Each such launch
+// costs about 4 us whatever its size (a few dozen blocks), and the fused
+// prologue's backward needs two sums: B8 T2048 C768, 4.8 + 3.9 -> 4.4 us,
+// the same bits
+__global__ __launch_bounds__(1024) void colsum2_kernel(ColSum a, ColSum b, int na) {
+  __shared__ float red[32][33];
+  const bool first = (int)blockIdx.x < na;
+  colsum_block(first ? a : b, first ? blockIdx.x : blockIdx.x - na, 0, red);
 }
 
 // column sums of a (np, n) array in one block row
@@ -845,9 +863,13 @@ hipError_t launch_qk_prologue(const QKArgs& args, int W, bool bwd, hipStream_t s
   if (!launched) return hipErrorInvalidValue;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !bwd) return e;
-  conv_grad_sums(a.part, a.dw, a.db, np, a.C, W, stream);
-  if ((e = hipGetLastError()) != hipSuccess || !a.nw || !a.dnw) return e;
-  colsum(a.npart, a.dnw, np * (int)grid.x, a.D, stream);
+  if (!a.nw || !a.dnw) {
+    conv_grad_sums(a.part, a.dw, a.db, np, a.C, W, stream);
+  } else {
+    const int nn = np * (int)grid.x, na = (n + 31) / 32;
+    colsum2_kernel<<<dim3(na + (a.D + 31) / 32), dim3(1024), 0, stream>>>(
+        ColSum{a.part, a.dw, np, n, np, W, a.db}, ColSum{a.npart, a.dnw, nn, a.D, nn, 0, nullptr}, na);
+  }
   return hipGetLastError();
 }
 
