@@ -179,6 +179,19 @@ int linatt_kata_bwd_onorm(const void* q, const void* k, const void* v, const flo
                           int H, int dk_dim, int dv_dim, int num_groups, float scale, int variant,
                           int dtype, void* stream);
 
+/* linatt_kata_bwd_onorm with the dk/dv pass split as in linatt_kata_bwd_split
+ * (not with the decayed score, whose pass has no split form).  workspace:
+ * linatt_kata_bwd_onorm_split_workspace_bytes bytes, 16-byte aligned (decay:
+ * whether c is given).  Same results up to the float32 summation order. */
+size_t linatt_kata_bwd_onorm_split_workspace_bytes(int B, int T, int HQ, int H, int dk_dim, int dv_dim,
+                                                   int num_groups, int variant, int decay, int dtype);
+int linatt_kata_bwd_onorm_split(const void* q, const void* k, const void* v, const float* c,
+                                const void* o, const float* den, const float* rstd,
+                                const float* norm_weight, const void* dy, void* dq, void* dk, void* dv,
+                                float* dc, float* dnorm_weight, void* workspace, size_t workspace_bytes,
+                                int B, int T, int HQ, int H, int dk_dim, int dv_dim, int num_groups,
+                                float scale, int variant, int dtype, void* stream);
+
 /* Size of the fixed device scratch behind linatt_kata_bwd_noalloc (32 MiB). */
 #define LINATT_NOALLOC_SCRATCH_BYTES (32u << 20)
 

@@ -53,6 +53,8 @@ SIGNATURES = {
     "linatt_kata_bwd_onorm_workspace_bytes": (_sz, [_i] * 5),
     "linatt_kata_fwd_num": (_i, [_vp] * 5 + [_i] * 7 + [_f, _i, _i, _vp]),
     "linatt_kata_bwd_onorm": (_i, [_vp] * 15 + [_i] * 7 + [_f, _i, _i, _vp]),
+    "linatt_kata_bwd_onorm_split_workspace_bytes": (_sz, [_i] * 10),
+    "linatt_kata_bwd_onorm_split": (_i, [_vp] * 15 + [_sz] + [_i] * 7 + [_f, _i, _i, _vp]),
     "linatt_delta_supported": (_i, [_i, _i, _i]),
     "linatt_delta_ctx_bytes": (_sz, [_i] * 6),
     "linatt_delta_bwd_workspace_bytes": (_sz, [_i] * 6),

@@ -473,14 +473,26 @@ size_t linatt_kata_bwd_onorm_workspace_bytes(int B, int T, int HQ, int dv_dim, i
   return onorm_part_offset(B, T, HQ, dv_dim, dtype) + nblk * dv_dim * sizeof(float);
 }
 
-int linatt_kata_bwd_onorm(const void* q, const void* k, const void* v, const float* c,
-                          const void* o, const float* den, const float* rstd,
-                          const float* norm_weight, const void* dy, void* dq, void* dk, void* dv,
-                          float* dc, float* dnorm_weight, void* workspace, int B, int T, int HQ,
-                          int H, int dk_dim, int dv_dim, int num_groups, float scale, int variant,
-                          int dtype, void* stream) {
+// where a split dk/dv pass's partial blocks start, behind the norm weight's partials
+static size_t onorm_split_offset(int B, int T, int HQ, int dv_dim, int dtype) {
+  return (linatt_kata_bwd_onorm_workspace_bytes(B, T, HQ, dv_dim, dtype) + 255) & ~(size_t)255;
+}
+// the decayed score's dk/dv pass has no split form
+static int onorm_split(int B, int T, int HQ, int H, int dk, int dv, int M, int variant, bool decay, int dtype) {
+  return decay ? 0 : bwd_split(B, T, HQ, H, dk, dv, M, variant, dtype);
+}
+static size_t onorm_split_ws(int B, int T, int HQ, int H, int dv, int L, int dtype) {
+  const size_t off = onorm_split_offset(B, T, HQ, dv, dtype);
+  return L ? off + kata_dkdv_part_bytes((int64_t)B * H, T, HQ / H, L) : off;
+}
+
+static int kata_bwd_onorm_entry(const char* fn, const void* q, const void* k, const void* v, const float* c,
+                                const void* o, const float* den, const float* rstd, const float* norm_weight,
+                                const void* dy, void* dq, void* dk, void* dv, float* dc, float* dnorm_weight,
+                                void* workspace, bool split, size_t ws_bytes, int B, int T, int HQ, int H,
+                                int dk_dim, int dv_dim, int num_groups, float scale, int variant, int dtype,
+                                void* stream) {
   g_last_error.clear();
-  const char* fn = "linatt_kata_bwd_onorm";
   int st = check_common(B, T, HQ, H, dk_dim, dv_dim, num_groups, scale, variant, dtype);
   if (st) return st;
   if ((st = check_onorm(fn, dk_dim, dv_dim, dtype, 0.f, true))) return st;
@@ -504,6 +516,14 @@ int linatt_kata_bwd_onorm(const void* q, const void* k, const void* v, const flo
   float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) +
                                          onorm_part_offset(B, T, HQ, dv_dim, dtype));
   a.nw_part = dnorm_weight ? part : nullptr;
+  if (split) {
+    a.split = onorm_split(B, T, HQ, H, dk_dim, dv_dim, num_groups, variant, c != nullptr, dtype);
+    if (a.split) {
+      if (ws_bytes < onorm_split_ws(B, T, HQ, H, dv_dim, a.split, dtype))
+        return fail(LINATT_EINVAL, std::string(fn) + ": workspace smaller than linatt_kata_bwd_onorm_split_workspace_bytes");
+      a.part = (float*)((char*)workspace + onorm_split_offset(B, T, HQ, dv_dim, dtype));
+    }
+  }
   bool found = false;
   hipError_t e = dispatch_bwd(a, KATA_BWD_DQ | KATA_BWD_DKDV, dtype, variant, c != nullptr,
                               (hipStream_t)stream, &found);
@@ -515,6 +535,35 @@ int linatt_kata_bwd_onorm(const void* q, const void* k, const void* v, const flo
   if (e != hipSuccess)
     return fail(LINATT_ELAUNCH, std::string(fn) + ": launch failed: " + hipGetErrorString(e));
   return LINATT_OK;
+}
+
+int linatt_kata_bwd_onorm(const void* q, const void* k, const void* v, const float* c,
+                          const void* o, const float* den, const float* rstd,
+                          const float* norm_weight, const void* dy, void* dq, void* dk, void* dv,
+                          float* dc, float* dnorm_weight, void* workspace, int B, int T, int HQ,
+                          int H, int dk_dim, int dv_dim, int num_groups, float scale, int variant,
+                          int dtype, void* stream) {
+  return kata_bwd_onorm_entry("linatt_kata_bwd_onorm", q, k, v, c, o, den, rstd, norm_weight, dy, dq, dk, dv, dc,
+                              dnorm_weight, workspace, false, 0, B, T, HQ, H, dk_dim, dv_dim, num_groups, scale,
+                              variant, dtype, stream);
+}
+
+size_t linatt_kata_bwd_onorm_split_workspace_bytes(int B, int T, int HQ, int H, int dk_dim, int dv_dim,
+                                                   int num_groups, int variant, int decay, int dtype) {
+  if (check_common(B, T, HQ, H, dk_dim, dv_dim, num_groups, 1.f, variant, dtype)) return 0;
+  return onorm_split_ws(B, T, HQ, H, dv_dim,
+                        onorm_split(B, T, HQ, H, dk_dim, dv_dim, num_groups, variant, decay != 0, dtype), dtype);
+}
+
+int linatt_kata_bwd_onorm_split(const void* q, const void* k, const void* v, const float* c,
+                                const void* o, const float* den, const float* rstd,
+                                const float* norm_weight, const void* dy, void* dq, void* dk, void* dv,
+                                float* dc, float* dnorm_weight, void* workspace, size_t workspace_bytes,
+                                int B, int T, int HQ, int H, int dk_dim, int dv_dim, int num_groups,
+                                float scale, int variant, int dtype, void* stream) {
+  return kata_bwd_onorm_entry("linatt_kata_bwd_onorm_split", q, k, v, c, o, den, rstd, norm_weight, dy, dq, dk, dv,
+                              dc, dnorm_weight, workspace, true, workspace_bytes, B, T, HQ, H, dk_dim, dv_dim,
+                              num_groups, scale, variant, dtype, stream);
 }
 
 int linatt_delta_supported(int dtype, int dk, int dv) { return delta_compiled(dtype, dk, dv) ? 1 : 0; }

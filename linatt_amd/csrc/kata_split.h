@@ -156,7 +156,8 @@ __host__ __device__ inline int64_t dkdv_part_offset(int piece, int nbk, int bh, 
 // Per 64-query tile of 128 keys, two workgroups per CU.  Unsplit -> split, us:
 // sum M = 2 B6 T1403 HQ12 H4 124 -> 105; concat M = 4 B1 H12 T2048 59 -> 47, B2
 // HQ16 H8 T2048 112 -> 86; M = 1 B1 HQ8 H4 T3000 108 -> 55; sum M = 4 B1 H12
-// T2048 141 -> 90.  Left unsplit: M = 1 B1 H8 T1500 (33 against 35), concat M = 4
+// T2048 141 -> 90; with the output norm, whole backward, B1 H12 T2048 concat M = 4
+// 111 -> 98, sum M = 4 268 -> 217.  Left unsplit: M = 1 B1 H8 T1500 (33 against 35), concat M = 4
 // B1 H4 T1000 (33 against 34).
 inline TileTime kata_dkdv_tile_time(int M, bool sum) {
   const double full = sum && M > 1 ? (M == 2 ? 3.2 : 7.0) : M == 1 ? 2.1 : M == 2 ? 2.3 : 2.8;

@@ -131,6 +131,11 @@ def _bwd_workspace_bytes(*args):
     return _lib.load().linatt_kata_bwd_workspace_bytes(*args)
 
 
+@functools.lru_cache(maxsize=256)
+def _bwd_onorm_workspace_bytes(*args):
+    return _lib.load().linatt_kata_bwd_onorm_split_workspace_bytes(*args)
+
+
 def parallel_kata_attn_fwd_impl(q, k, v, num_groups, scale, bT, bK, c=None):
     """Concat-SPD causal forward; returns ``(o, den)``
     (reference ``kata/parallel_kata_attn.py:211-288``).  ``c`` is an optional
@@ -304,7 +309,7 @@ def _onorm_fused(dtype, dk, dv, need_grad):
 
 class _KataONormFunction(torch.autograd.Function):
     """y = RMSNorm(KATA(q, k, v)) per (b, t, head) row: ``linatt_kata_fwd_onorm``
-    writes o, den, y and rstd in one forward; ``linatt_kata_bwd_onorm`` forms
+    writes o, den, y and rstd in one forward; ``linatt_kata_bwd_onorm_split`` forms
     the norm's dO from dy inside the dq pass and sums the weight gradient."""
 
     @staticmethod
@@ -349,13 +354,13 @@ class _KataONormFunction(torch.autograd.Function):
         dc = torch.empty_like(cf) if cf is not None else None
         dw = torch.empty(dv, device=q.device, dtype=torch.float32) if w is not None else None
         L = _lib.load()
-        ws = torch.empty(L.linatt_kata_bwd_onorm_workspace_bytes(B, T, HQ, dv, _lib.dtype_code(v.dtype)),
-                         device=q.device, dtype=torch.uint8)
-        _lib.check("linatt_kata_bwd_onorm", L.linatt_kata_bwd_onorm(
+        shape, code, var = (B, T, HQ, H, dk, dv, num_groups), _lib.dtype_code(v.dtype), _VARIANT[variant]
+        nws = _bwd_onorm_workspace_bytes(*shape, var, int(cf is not None), code)
+        ws = torch.empty(nws, device=q.device, dtype=torch.uint8)
+        _lib.check("linatt_kata_bwd_onorm_split", L.linatt_kata_bwd_onorm_split(
             _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(cf), _lib.ptr(o), _lib.ptr(den),
             _lib.ptr(rstd), _lib.ptr(w), _lib.ptr(dy), _lib.ptr(dq), _lib.ptr(dk_), _lib.ptr(dv_),
-            _lib.ptr(dc), _lib.ptr(dw), _lib.ptr(ws), B, T, HQ, H, dk, dv, num_groups, scale,
-            _VARIANT[variant], _lib.dtype_code(v.dtype), _lib.stream_of(q)))
+            _lib.ptr(dc), _lib.ptr(dw), _lib.ptr(ws), nws, *shape, scale, var, code, _lib.stream_of(q)))
         qd, kd, vd, cd, wd = ctx.dtypes
         return (_lib.as_dtype(dq, qd), _lib.as_dtype(dk_, kd), _lib.as_dtype(dv_, vd),
                 _lib.as_dtype(dc, cd) if dc is not None else None,

@@ -108,3 +108,48 @@ def test_split_backward_equals_unsplit(B, T, HQ, H, M, variant):
         print("  rel %.1e" % ((a - b).norm() / a.norm()).item(), flush=True)
         assert (a - b).norm() <= 2.0 ** -8 * a.norm()
         assert ((a - b).abs() <= 2.0 ** -7 * a.abs() + 2.0 ** -12 * a.abs().max()).all()
+
+
+@pytest.mark.parametrize("B,T,HQ,H,M,variant,decay", [(1, 2048, 12, 12, 4, "concat", False), (1, 2100, 4, 1, 1, "concat", False),
+                                                      (1, 1930, 3, 3, 4, "sum", False), (1, 300, 2, 2, 2, "concat", True)])
+def test_split_onorm_backward_equals_unsplit(B, T, HQ, H, M, variant, decay):
+    """The same with the output norm in the dq pass (the decayed score: never
+    split).  dq, dc and the weight's gradient come from the same launches."""
+    from linatt_amd import _lib
+    print(f"\nsplit onorm backward B{B} T{T} HQ{HQ} H{H} M{M} {variant} decay={decay}", flush=True)
+    L, p = _lib.load(), _lib.ptr
+    g = torch.Generator().manual_seed(T + M)
+    q, dy = (torch.randn(B, T, HQ, 64, generator=g).bfloat16().cuda() for _ in range(2))
+    k, v = (torch.randn(B, T, H, 64, generator=g).bfloat16().cuda() for _ in range(2))
+    w = (torch.rand(64, generator=g) + 0.5).cuda()
+    c = (-torch.rand(B, T, HQ, generator=g) * 0.05).cumsum(1).cuda() if decay else None
+    o, y = torch.empty_like(q), torch.empty_like(q)
+    den, rstd = (torch.empty(B, T, HQ, device="cuda") for _ in range(2))
+    var, sp, sc, shape = int(variant == "sum"), _lib.stream_of(q), math.sqrt(M) / 8, (B, T, HQ, H, 64, 64, M)
+    _lib.check("fwd", L.linatt_kata_fwd_onorm(p(q), p(k), p(v), p(c), p(o), p(den), p(w), 1e-5, p(y), p(rstd), *shape,
+                                              sc, var, 1, sp))
+    nb = L.linatt_kata_bwd_onorm_workspace_bytes(B, T, HQ, 64, 1)
+    ns = L.linatt_kata_bwd_onorm_split_workspace_bytes(*shape, var, int(decay), 1)
+    assert (ns > nb + 256) == (not decay)
+    ws = torch.empty(ns, device="cuda", dtype=torch.uint8)
+    out = []
+    for split in (False, True):
+        gr = [torch.full_like(x, float("nan")) for x in (q, w, k, v)] + ([torch.full_like(c, float("nan"))] if decay else [])
+        dq, dw, dk, dv = gr[:4]
+        dc = gr[4] if decay else None
+        head = (p(q), p(k), p(v), p(c), p(o), p(den), p(rstd), p(w), p(dy), p(dq), p(dk), p(dv), p(dc), p(dw), p(ws))
+        tail = (*shape, sc, var, 1, sp)
+        if split:
+            _lib.check("split", L.linatt_kata_bwd_onorm_split(*head, ns, *tail))
+        else:
+            _lib.check("bwd", L.linatt_kata_bwd_onorm(*head, *tail))
+        out.append(gr)
+    if not decay:
+        assert L.linatt_kata_bwd_onorm_split(*head, ns - 1, *tail) == -1
+    torch.cuda.synchronize()
+    assert all(torch.equal(out[0][i], out[1][i]) for i in (0, 1))
+    for a, b in zip(out[0][2:4], out[1][2:4]):
+        a, b = a.double(), b.double()
+        print("  rel %.1e" % ((a - b).norm() / a.norm()).item(), flush=True)
+        assert (a - b).norm() <= 2.0 ** -8 * a.norm()
+        assert ((a - b).abs() <= 2.0 ** -7 * a.abs() + 2.0 ** -12 * a.abs().max()).all()
