@@ -1274,32 +1274,37 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
   }
 }
 
-// The split dk/dv pass's outputs where the list was cut: a wave per 32 keys,
-// the pieces added in order, stored as the unsplit kernel stores its registers.
+// The split dk/dv pass's outputs where the list was cut, the pieces added in
+// order, stored as the unsplit kernel stores its registers.  As the forward's:
+// a workgroup per 32 keys, waves 0 and 1 half of dv's register quads each,
+// waves 2 and 3 dk's, four pieces' loads in flight (a wave per 32 keys: sum
+// M = 2 B1 H8 T2048 backward 89 us, now 82; M = 1 B1 HQ8 H4 T3000 108, now 97).
 template <typename T, bool K16>
 __global__ __launch_bounds__(256) void kata_dkdv_split_finish_kernel(const float* __restrict__ part, T* __restrict__ dk,
                                                                      T* __restrict__ dv, int Tn, int H, int G, int nkt,
                                                                      int nbk, int split) {
   const int lane = threadIdx.x & 63, cl = lane & 31, hh = lane >> 5, w = wave_id();
-  const int st = blockIdx.x % nkt, bh = blockIdx.x / nkt;
+  const int blk = blockIdx.x & 3, st = (blockIdx.x >> 2) % nkt, bh = (blockIdx.x >> 2) / nkt;
   const int pieces = split_pieces(kata_query_tiles(st, Tn, G), split);
-  if (pieces == 1) return;
-  f32x4 x[16] = {};
+  const int sw = 128 * st + 32 * blk;
+  if (pieces == 1 || sw >= Tn) return;
+  f32x4 x[4] = {};
+#pragma unroll 4
   for (int i = 0; i < pieces; ++i) {
-    const float* p = part + dkdv_part_offset(i, nbk, bh, nkt, 4 * st + w) + 4 * lane;
+    const float* p = part + dkdv_part_offset(i, nbk, bh, nkt, 4 * st + blk) + 4 * lane;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) x[e] += *reinterpret_cast<const f32x4*>(p + 256 * e);
+    for (int j = 0; j < 4; ++j) x[j] += *reinterpret_cast<const f32x4*>(p + 256 * (4 * w + j));
   }
-  const int sw = 128 * st + 32 * w;
   const int64_t row0 = (int64_t)(bh / H) * Tn * H + bh % H;
   auto out = [&](T* base, int s, int d, const f32x4& y, float f) __attribute__((always_inline)) {
     if (s < Tn) st4<T>(base + (row0 + (int64_t)s * H) * 64 + d, to4<T>(y[0] * f, y[1] * f, y[2] * f, y[3] * f));
   };
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    out(dv, sw + cl, 8 * e + 4 * hh, x[e], 1.f);
-    if constexpr (K16) out(dk, sw + 16 * (e & 1) + (lane & 15), 16 * (e >> 1) + 4 * (lane >> 4), x[8 + e], 2.f);
-    else out(dk, sw + cl, 8 * e + 4 * hh, x[8 + e], 2.f);
+  for (int j = 0; j < 4; ++j) {
+    const int e = 4 * (w & 1) + j;
+    if (w < 2) out(dv, sw + cl, 8 * e + 4 * hh, x[j], 1.f);
+    else if constexpr (K16) out(dk, sw + 16 * (e & 1) + (lane & 15), 16 * (e >> 1) + 4 * (lane >> 4), x[j], 2.f);
+    else out(dk, sw + cl, 8 * e + 4 * hh, x[j], 2.f);
   }
 }
 
@@ -1355,7 +1360,7 @@ hipError_t launch_kata_bwd(const KataArgs& a, int parts, hipStream_t stream) {
         } else if constexpr (__is_same(T, __bf16) && DK == 64 && !DECAY) {
           const int G = a.HQ / a.H;
           go(BoolC<true>{}, kata_dkdv_items(a.T, G, a.split) * nbk);
-          kata_dkdv_split_finish_kernel<T, DK / M == 16><<<dim3(nkt * nbk), dim3(256), 0, stream>>>(
+          kata_dkdv_split_finish_kernel<T, DK / M == 16><<<dim3(4 * nkt * nbk), dim3(256), 0, stream>>>(
               a.part, (T*)a.dk, (T*)a.dv, a.T, a.H, G, nkt, nbk, a.split);
         } else {
           return hipErrorInvalidValue;

@@ -49,33 +49,38 @@ __host__ __device__ inline int64_t fwd_part_offset(int piece, int nbh, int bh, i
   return (((int64_t)piece * nbh + bh) * (4 * nqt) + blk) * kFwdPart;
 }
 
-// The split launch's outputs where the key list was cut: a wave per 32
-// queries, the pieces added in order.
+// The split launch's outputs where the key list was cut, the pieces added in
+// order.  Latency-bound (up to kMaxPieces dependent adds behind their loads), so
+// a workgroup takes one block of 32 queries, wave w its register quads 2w and
+// 2w + 1, and eight pieces' loads are in flight.  With a workgroup per 128
+// queries and a wave per block, the call took: float32 B1 H4 T512 19.6 us, now
+// 17.0; fp16 M = 2 B1 H12 T3001 40.1, now 37.0.
 template <typename T>
 __global__ __launch_bounds__(256) void kata_fwd_split_finish_kernel(const float* __restrict__ part, T* __restrict__ o,
                                                                     float* __restrict__ den, int Tn, int HQ, int nqt,
                                                                     int nbh, float scale2, int split) {
   const int lane = threadIdx.x & 63, cl = lane & 31, hh = lane >> 5;
-  const int qt = blockIdx.x % nqt, bh = blockIdx.x / nqt, w = wave_id();
+  const int blk = blockIdx.x & 3, qt = (blockIdx.x >> 2) % nqt, bh = (blockIdx.x >> 2) / nqt, w = wave_id();
   const int pieces = split_pieces(kata_key_tiles(qt, Tn), split);
-  if (pieces == 1) return;
-  f32x4 x[8] = {};
+  const int t0 = 128 * qt + 32 * blk;
+  if (pieces == 1 || t0 >= Tn) return;
+  f32x4 x[2] = {};
   float dsum = 0.f;
-#pragma unroll 2
+#pragma unroll 8
   for (int i = 0; i < pieces; ++i) {
-    const float* p = part + fwd_part_offset(i, nbh, bh, nqt, 4 * qt + w);
+    const float* p = part + fwd_part_offset(i, nbh, bh, nqt, 4 * qt + blk);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] += *reinterpret_cast<const f32x4*>(p + 256 * e + 4 * lane);
+    for (int j = 0; j < 2; ++j) x[j] += *reinterpret_cast<const f32x4*>(p + 256 * (2 * w + j) + 4 * lane);
     dsum += p[2048 + lane];
   }
-  const int tl = 128 * qt + 32 * w + cl;
+  const int tl = t0 + cl;
   if (tl >= Tn) return;
   const float inv = dsum > 0.f ? 1.f / dsum : 1.f;
   const int64_t row = ((int64_t)(bh / HQ) * Tn + tl) * HQ + bh % HQ;
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
-    st4<T>(o + row * 64 + 8 * e + 4 * hh, to4<T>(x[e][0] * inv, x[e][1] * inv, x[e][2] * inv, x[e][3] * inv));
-  if (hh == 0) den[row] = dsum * scale2;
+  for (int j = 0; j < 2; ++j)
+    st4<T>(o + row * 64 + 8 * (2 * w + j) + 4 * hh, to4<T>(x[j][0] * inv, x[j][1] * inv, x[j][2] * inv, x[j][3] * inv));
+  if (hh == 0 && w == 0) den[row] = dsum * scale2;
 }
 
 // SPLIT: the workgroup's share of a split launch (kata_split.h)
@@ -612,7 +617,7 @@ hipError_t launch_kata_fwd(const KataArgs& a, hipStream_t stream) {
     if (a.split) grid.x = kata_fwd_items(a.T, a.split) * nbh;
     auto finish = [&]() {
       if (!a.split) return;
-      kata_fwd_split_finish_kernel<T><<<dim3(nqt * nbh), block, 0, stream>>>(
+      kata_fwd_split_finish_kernel<T><<<dim3(4 * nqt * nbh), block, 0, stream>>>(
           a.part, (T*)a.o, a.den, a.T, a.HQ, nqt, nbh, a.scale * a.scale, a.split);
     };
     if constexpr (sizeof(T) == 2 && (DK == 64 || DK == 128) && DV == 64) {
