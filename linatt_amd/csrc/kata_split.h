@@ -102,8 +102,8 @@ inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileT
 // three workgroups per CU at dk = 64, two at dk = 128; fp16 adds the row
 // rescaling.  float32: 32 x 32 x 2 products, two workgroups per CU.
 // Unsplit -> split, us: float32 B1 H4 T512 48 -> 17; fp16 M = 2 B1 H12 T3001
-// 57 -> 37; bf16 (with a second launch 3 us slower than now) B1 H12 T2048: sum M = 4 76 -> 40, decayed dk = 128 55 -> 33,
-// concat M = 4 28 -> 26.  Left unsplit: concat M = 4 at B2 T2048 (30 against 33),
+// 57 -> 37; bf16 (with a second launch 3 us slower than now) B1 H12 T2048: sum
+// M = 4 76 -> 40, decayed dk = 128 55 -> 33, concat M = 4 28 -> 26.  Left unsplit: concat M = 4 at B2 T2048 (30 against 33),
 // B4 (39 against 51), M = 1 at B1 T1500 (18 against 19).
 inline TileTime kata_fwd_tile_time(int elt_bytes, bool fp16, int dk, int M, bool sum, bool decay) {
   if (elt_bytes == 4) return {6., 14., 512, 8.};
@@ -153,13 +153,13 @@ constexpr int kDkdvPart = 32 * 128;
 __host__ __device__ inline int64_t dkdv_part_offset(int piece, int nbk, int bh, int nkt, int blk) {
   return (((int64_t)piece * nbk + bh) * (4 * nkt) + blk) * kDkdvPart;
 }
-// Per 64-query tile of 128 keys, two workgroups per CU.  Unsplit -> split, us:
+// Per 64-query tile of 128 keys, two workgroups per CU.  Unsplit -> split, us
+// (with a second launch 5 to 10 us slower than now):
 // sum M = 2 B6 T1403 HQ12 H4 124 -> 105; concat M = 4 B1 H12 T2048 59 -> 47, B2
 // HQ16 H8 T2048 112 -> 86; M = 1 B1 HQ8 H4 T3000 108 -> 55; sum M = 4 B1 H12
 // T2048 141 -> 90; with the output norm, whole backward, B1 H12 T2048 concat M = 4
-// 111 -> 93, sum M = 4 268 -> 209 (the first figures of the list: with a second
-// launch 5 to 10 us slower than now).  Left unsplit: M = 1 B1 H8 T1500 (33 against 35), concat M = 4
-// B1 H4 T1000 (33 against 34).
+// 111 -> 98, sum M = 4 268 -> 217 (now 93 and 209).  Left unsplit: M = 1 B1 H8
+// T1500 (33 against 35), concat M = 4 B1 H4 T1000 (33 against 34).
 inline TileTime kata_dkdv_tile_time(int M, bool sum) {
   const double full = sum && M > 1 ? (M == 2 ? 3.2 : 7.0) : M == 1 ? 2.1 : M == 2 ? 2.3 : 2.8;
   return {full / 1.6, full, 512, 13.};
