@@ -38,3 +38,20 @@ def test_l2norm_fwd_bwd(n, d, shift, dtype):
     yr, gr = y.detach().double(), dy.double()
     ref = r * (gr - yr * (yr * gr).sum(-1, keepdim=True))
     assert (dx.double() - ref).abs().max() <= BOUND[dtype] * ref.abs().max()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,d", [(1, 64), (6000, 64), (3001, 128), (1501, 256)])
+def test_l2norm_bits_independent_of_alignment(n, d, dtype):
+    """The row-group kernels keep the general kernel's summation order: the
+    same values at 16-byte aligned and at other addresses give the same bits."""
+    from linatt_amd.delta_rule import l2norm
+    g = torch.Generator().manual_seed(n + d)
+    x, dy = (torch.randn(n, d, generator=g).to(dtype) for _ in range(2))
+    out = []
+    for shift in (0, 1):
+        xs = _at(x, shift).requires_grad_(True)
+        y = l2norm(xs, 1e-6)
+        out.append((y, *torch.autograd.grad(y, xs, _at(dy, shift))))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
