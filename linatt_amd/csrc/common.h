@@ -83,6 +83,18 @@ __device__ __forceinline__ void st4(T* p, v4_t<T> v) {
   }
 }
 
+// 8 contiguous elements at a 16-byte aligned address (fp32: two 16-byte stores;
+// an 8-float vector access would assume 32)
+template <typename T>
+__device__ __forceinline__ void st8(T* p, v8_t<T> v) {
+  if constexpr (sizeof(T) == 2) {
+    *reinterpret_cast<uint4*>(p) = __builtin_bit_cast(uint4, v);
+  } else {
+    reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
+    reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ v8_t<T> cat44(v4_t<T> a, v4_t<T> b) {
   return v8_t<T>{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};

@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void l2norm_fwd_rows_kernel(const T* __restric
       float a[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) a[j] = (float)xv[i][k][j];
-      if (row < n) *reinterpret_cast<v8_t<T>*>(y + (int64_t)row * D + 64 * k + c8) = l2_out<T, K>(a, r);
+      if (row < n) st8<T>(y + (int64_t)row * D + 64 * k + c8, l2_out<T, K>(a, r));
     }
     if (row < n && sub == 0) rstd[row] = r;
   }
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void l2norm_bwd_rows_kernel(const T* __restric
       float a[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) a[j] = fmaf(-(float)yv[i][k][j], dot, (float)gv[i][k][j]);
-      if (row < n) *reinterpret_cast<v8_t<T>*>(dx + (int64_t)row * D + 64 * k + c8) = l2_out<T, K>(a, rs[i]);
+      if (row < n) st8<T>(dx + (int64_t)row * D + 64 * k + c8, l2_out<T, K>(a, rs[i]));
     }
   }
 }

@@ -55,3 +55,27 @@ def test_l2norm_bits_independent_of_alignment(n, d, dtype):
         out.append((y, *torch.autograd.grad(y, xs, _at(dy, shift))))
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_l2norm_float32_outputs_at_16_mod_32(d):
+    """float32 outputs at addresses that are 16-byte but not 32-byte aligned
+    take the row-group kernels too: the same bits as at 32-byte aligned ones,
+    and nothing outside them is written."""
+    from linatt_amd import _lib
+    L, p, n = _lib.load(), _lib.ptr, 67
+    g = torch.Generator().manual_seed(d)
+    x, dy = (torch.randn(n, d, generator=g).cuda() for _ in range(2))
+    out, sp = [], _lib.stream_of(x)
+    for off in (8, 4):
+        bufs = [torch.full((n * d + 16,), float("nan"), device="cuda") for _ in range(2)]
+        assert all(b.data_ptr() % 32 == 0 for b in bufs)
+        y, dx = (b[off:off + n * d].view(n, d) for b in bufs)
+        rstd = torch.empty(n, device="cuda")
+        _lib.check("fwd", L.linatt_l2norm_fwd(p(x), p(y), p(rstd), n, d, 1e-6, 0, sp))
+        _lib.check("bwd", L.linatt_l2norm_bwd(p(y), p(rstd), p(dy), p(dx), n, d, 0, sp))
+        for b in bufs:
+            assert b[:off].isnan().all() and b[off + n * d:].isnan().all() and not b[off:off + n * d].isnan().any()
+        out.append((y, rstd, dx))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
