@@ -325,12 +325,11 @@ static int kata_bwd_entry(const char* fn, int parts, const void* q, const void* 
   a.c = c;
   a.dc = dc;
   if (split) {
+    // the size also covers the pass's own arrays, which an unsplit launch writes too
     a.split = bwd_split(B, T, HQ, H, dk_dim, dv_dim, num_groups, variant, dtype);
-    if (a.split) {
-      if (ws_bytes < bwd_split_ws(B, T, HQ, H, dv_dim, a.split, dtype))
-        return fail(LINATT_EINVAL, std::string(fn) + ": workspace smaller than linatt_kata_bwd_split_workspace_bytes");
-      a.part = (float*)((char*)workspace + bwd_part_offset(B, T, HQ, dv_dim, dtype));
-    }
+    if (ws_bytes < bwd_split_ws(B, T, HQ, H, dv_dim, a.split, dtype))
+      return fail(LINATT_EINVAL, std::string(fn) + ": workspace smaller than linatt_kata_bwd_split_workspace_bytes");
+    if (a.split) a.part = (float*)((char*)workspace + bwd_part_offset(B, T, HQ, dv_dim, dtype));
   }
   bool found = false;
   hipError_t e = dispatch_bwd(a, parts, dtype, variant, c != nullptr, (hipStream_t)stream, &found);
@@ -518,11 +517,9 @@ static int kata_bwd_onorm_entry(const char* fn, const void* q, const void* k, co
   a.nw_part = dnorm_weight ? part : nullptr;
   if (split) {
     a.split = onorm_split(B, T, HQ, H, dk_dim, dv_dim, num_groups, variant, c != nullptr, dtype);
-    if (a.split) {
-      if (ws_bytes < onorm_split_ws(B, T, HQ, H, dv_dim, a.split, dtype))
-        return fail(LINATT_EINVAL, std::string(fn) + ": workspace smaller than linatt_kata_bwd_onorm_split_workspace_bytes");
-      a.part = (float*)((char*)workspace + onorm_split_offset(B, T, HQ, dv_dim, dtype));
-    }
+    if (ws_bytes < onorm_split_ws(B, T, HQ, H, dv_dim, a.split, dtype))
+      return fail(LINATT_EINVAL, std::string(fn) + ": workspace smaller than linatt_kata_bwd_onorm_split_workspace_bytes");
+    if (a.split) a.part = (float*)((char*)workspace + onorm_split_offset(B, T, HQ, dv_dim, dtype));
   }
   bool found = false;
   hipError_t e = dispatch_bwd(a, KATA_BWD_DQ | KATA_BWD_DKDV, dtype, variant, c != nullptr,

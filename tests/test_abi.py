@@ -165,6 +165,33 @@ def test_bwd_argument_errors(lib):
     assert f(dk=64, M=5) == EINVAL
 
 
+@pytest.mark.parametrize("B,T,HQ,H,dk,M,variant,dtype,decay", [
+    (8, 2048, 12, 12, 64, 4, 0, 1, 0), (1, 100, 2, 2, 64, 4, 0, 1, 0), (2, 300, 4, 2, 64, 2, 1, 2, 0),
+    (1, 300, 2, 2, 64, 2, 0, 0, 0), (2, 2048, 4, 4, 128, 2, 0, 1, 0), (8, 2048, 16, 16, 64, 2, 0, 1, 1),
+    (1, 2048, 12, 12, 64, 2, 0, 1, 1), (1, 2048, 12, 12, 64, 4, 0, 1, 0)])
+def test_bwd_split_workspace_size_checked(lib, B, T, HQ, H, dk, M, variant, dtype, decay):
+    """The split entries refuse a workspace smaller than their query names,
+    before any launch, whether the call splits (the last shape) or not: an
+    unsplit backward writes its own arrays there all the same."""
+    shape = (B, T, HQ, H, dk, 64, M)
+    sc = 0.25
+    if not decay:
+        need = lib.linatt_kata_bwd_split_workspace_bytes(*shape, variant, dtype)
+        assert need >= lib.linatt_kata_bwd_workspace_bytes(B, T, HQ, 64, dtype) > 0
+        for n in (0, need - 1):
+            assert lib.linatt_kata_bwd_split(*[FAKE] * 10, n, *shape, sc, variant, dtype, None) == -1
+            assert b"workspace smaller" in lib.linatt_last_error()
+    if dtype != 1 or dk != 64:
+        return  # the output norm's backward runs there only
+    need = lib.linatt_kata_bwd_onorm_split_workspace_bytes(*shape, variant, decay, dtype)
+    assert need >= lib.linatt_kata_bwd_onorm_workspace_bytes(B, T, HQ, 64, dtype) > 0
+    c = FAKE if decay else None
+    for n in (0, need - 1):
+        assert lib.linatt_kata_bwd_onorm_split(FAKE, FAKE, FAKE, c, *[FAKE] * 8, c, FAKE, FAKE, n, *shape, sc, variant,
+                                               dtype, None) == -1
+        assert b"workspace smaller" in lib.linatt_last_error()
+
+
 def test_python_layer_rejects_cpu_tensors(lib):
     import torch
     from linatt_amd import parallel_kata_attn as P
