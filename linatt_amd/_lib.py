@@ -157,8 +157,10 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_of(t: torch.Tensor) -> int:
-    """Current HIP stream of the tensor's device, as an address."""
-    if _raw_stream is not None:
+    """Current HIP stream of the tensor's device, as an address; a tensor that
+    is not on a GPU raises (the raw call would answer with the current
+    device's stream, and a kernel would be launched on host addresses)."""
+    if _raw_stream is not None and t.is_cuda:
         return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 

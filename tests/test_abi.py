@@ -200,6 +200,23 @@ def test_python_layer_rejects_cpu_tensors(lib):
         P.parallel_kata_attn_fwd(q, q, q)
 
 
+def test_stream_of_refuses_cpu_tensors(monkeypatch):
+    """No call reaches a launch with a CPU tensor, an autograd function applied
+    directly (past the public call's own check) included."""
+    import torch
+    from linatt_amd import _lib, delta_rule
+    monkeypatch.setattr(_lib, "_raw_stream", lambda device: 0)
+    q = torch.randn(1, 4, 1, 64, dtype=torch.bfloat16)
+    with pytest.raises((ValueError, RuntimeError)):
+        _lib.stream_of(q)
+    # the C entry is never reached: its answer would be a LinattError
+    for call in (lambda: delta_rule._L2Norm.apply(q, 1e-6),
+                 lambda: delta_rule.ChunkDeltaRuleFunction.apply(q, q, q, torch.rand(1, 4, 1), None, 1.0, None, False)):
+        with pytest.raises((ValueError, RuntimeError)) as e:
+            call()
+        assert not isinstance(e.value, _lib.LinattError)
+
+
 def test_noalloc_rejects_oversized_before_device_work(lib):
     EINVAL = -1
     assert lib.linatt_noalloc_scratch_bytes() == 32 << 20
