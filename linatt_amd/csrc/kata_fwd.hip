@@ -32,17 +32,20 @@ namespace linatt {
 // One piece's unnormalised sums of a wave's 32 queries, in register order (lane
 // l's 16 bytes i at 256 i + 4 l: whole 1 KiB runs per store, and the finish
 // kernel loads them back the same way; rows of o order instead scattered each
-// store over 32 rows and cost 10 to 25 us a call).  f undoes the fp16 row scale.
-template <int DV>
-__device__ __forceinline__ void store_fwd_partial(float* p, const f32x16 (&oacc)[DV / 32], float dsum, float f, int lane) {
+// store over 32 rows and cost 10 to 25 us a call).  float16: in units of the
+// row scale pe, stored beside the sum that both lane halves hold (taken out of
+// the sums here, a row of decayed weights below 2^-128 had a denormal sum with
+// an infinite reciprocal).
+template <typename T, int DV>
+__device__ __forceinline__ void store_fwd_partial(float* p, const f32x16 (&oacc)[DV / 32], float dsum, float pe, int lane) {
   static_assert(DV == 64, "32 x 64 blocks");
 #pragma unroll
   for (int db = 0; db < 2; ++db)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       *reinterpret_cast<f32x4*>(p + 256 * (4 * db + i) + 4 * lane) =
-          f32x4{oacc[db][4 * i] * f, oacc[db][4 * i + 1] * f, oacc[db][4 * i + 2] * f, oacc[db][4 * i + 3] * f};
-  p[2048 + lane] = dsum * f;
+          f32x4{oacc[db][4 * i], oacc[db][4 * i + 1], oacc[db][4 * i + 2], oacc[db][4 * i + 3]};
+  p[2048 + lane] = __is_same(T, _Float16) && lane >= 32 ? pe : dsum;
 }
 // block `blk` (32 queries) of head bh, piece `piece`
 __host__ __device__ inline int64_t fwd_part_offset(int piece, int nbh, int bh, int nqt, int blk) {
@@ -66,13 +69,34 @@ __global__ __launch_bounds__(256) void kata_fwd_split_finish_kernel(const float*
   if (pieces == 1 || t0 >= Tn) return;
   f32x4 x[2] = {};
   float dsum = 0.f;
+  // float16: the sums so far are in units of 2^es, the smallest of the pieces'
+  // scales (the unsplit kernel's running one); a piece of zero weights has none
+  constexpr bool kRescale = __is_same(T, _Float16);
+  constexpr int kNone = 1000;
+  int es = kNone;
 #pragma unroll 8
   for (int i = 0; i < pieces; ++i) {
     const float* p = part + fwd_part_offset(i, nbh, bh, nqt, 4 * qt + blk);
+    if constexpr (kRescale) {
+      const float d = p[2048 + cl];
+      const int e = (int)(__float_as_uint(p[2080 + cl]) >> 23) - 127;
+      const int en = d == 0.f ? es : min(es, e);
+      const int sx = en - es, sp = d == 0.f ? 0 : en - e;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) x[j] += *reinterpret_cast<const f32x4*>(p + 256 * (2 * w + j) + 4 * lane);
-    dsum += p[2048 + lane];
+      for (int j = 0; j < 2; ++j) {
+        const f32x4 y = *reinterpret_cast<const f32x4*>(p + 256 * (2 * w + j) + 4 * lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[j][r] = ldexpf(x[j][r], sx) + ldexpf(y[r], sp);
+      }
+      dsum = ldexpf(dsum, sx) + ldexpf(d, sp);
+      es = en;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) x[j] += *reinterpret_cast<const f32x4*>(p + 256 * (2 * w + j) + 4 * lane);
+      dsum += p[2048 + lane];
+    }
   }
+  if (kRescale && es != kNone) scale2 = ldexpf(scale2, -es);
   const int tl = t0 + cl;
   if (tl >= Tn) return;
   const float inv = dsum > 0.f ? 1.f / dsum : 1.f;
@@ -241,7 +265,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void kata_fwd_kernel(
   const float dsum = dpart + __shfl_xor(dpart, 32);
   if constexpr (SPLIT) {
     if (run.pieces > 1) {
-      store_fwd_partial<DV>(part + fwd_part_offset(run.piece, nbh, bh, nqt, 4 * qt + w), oacc, dsum, 1.f / pe, lane);
+      store_fwd_partial<T, DV>(part + fwd_part_offset(run.piece, nbh, bh, nqt, 4 * qt + w), oacc, dsum, pe, lane);
       return;
     }
   }
@@ -538,8 +562,7 @@ __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void kata_fwd_tile_kernel(
   const float dsum = dpart + __shfl_xor(dpart, 32);
   if constexpr (EPI == 3) {
     if (run.pieces > 1) {
-      store_fwd_partial<DV>(on.part + fwd_part_offset(run.piece, nbh, bh, nqt, 4 * qt + w), oacc, dsum, 1.f / pe,
-                            lane);
+      store_fwd_partial<T, DV>(on.part + fwd_part_offset(run.piece, nbh, bh, nqt, 4 * qt + w), oacc, dsum, pe, lane);
       return;
     }
   }

@@ -49,7 +49,8 @@ __device__ __forceinline__ SplitRun kata_fwd_run(int j, int nqt, int T, int L) {
   return r;
 }
 
-// floats of a partial block of 32 queries: 32 x 64 sums, a den per lane
+// floats of a partial block of 32 queries: 32 x 64 sums, a den per lane (float16:
+// per lane of the lower half, the row scale in the upper)
 constexpr int kFwdPart = 32 * 64 + 64;
 // most pieces of one list (the partial blocks reserved for it)
 constexpr int kMaxPieces = 16;

@@ -56,6 +56,43 @@ def test_split_forward_equals_unsplit(B, T, HQ, H, dk, M, variant, decay, dtype)
     assert ((o1 - o2).abs() <= SPACING[dtype] * o1.abs() + 2 * acc * v.double().abs().max()).all()
 
 
+def test_split_forward_fp16_tiny_weights():
+    """float16 rows whose every weight lies below 2^-128 (four small keys, then
+    a decay of e^-84.5 and zero keys): the row scale keeps them through the
+    pieces, as in the unsplit kernel.  The four weights are equal, so o is the
+    mean of their v rows to one float16 spacing."""
+    from linatt_amd import _lib
+    L, p = _lib.load(), _lib.ptr
+    B, T, H, dk, M = 1, 3100, 2, 64, 2
+    print(f"\nsplit forward, weights below 2^-128, B{B} T{T} H{H}", flush=True)
+    q = torch.full((B, T, H, dk), 2.0 ** -5, dtype=torch.float16, device="cuda")
+    k = torch.zeros_like(q)
+    k[:, :4] = 2.0 ** -5
+    v = torch.randn(B, T, H, 64, generator=torch.Generator().manual_seed(0)).half().cuda()
+    c = torch.zeros(B, T, H, device="cuda")
+    c[:, 64:] = -84.5
+    shape = (B, T, H, H, dk, 64, M)
+    nws = L.linatt_kata_fwd_workspace_bytes(*shape, 0, 1, 2)
+    assert nws > 0
+    ws = torch.empty(nws, device="cuda", dtype=torch.uint8)
+    out = []
+    for split in (False, True):
+        o, den = torch.full_like(v, float("nan")), torch.full((B, T, H), float("nan"), device="cuda")
+        head, tail = (p(q), p(k), p(v), p(c), p(o), p(den)), (*shape, 1.0, 0, 2, _lib.stream_of(q))
+        if split:
+            _lib.check("split", L.linatt_kata_fwd_split(*head, p(ws), nws, *tail))
+        else:
+            _lib.check("fwd", L.linatt_kata_fwd(*head, *tail))
+        out.append((o.double(), den.double()))
+    torch.cuda.synchronize()
+    (o1, d1), (o2, d2) = out
+    assert 0 < d1[:, 64:].max() < 2.0 ** -128
+    mean = v[:, :4].double().mean(1, keepdim=True)
+    for o in (o1, o2):
+        assert ((o[:, 64:] - mean).abs() <= 2.0 ** -10 * mean.abs() + 2.0 ** -24).all()
+    assert torch.equal(d1, d2) and torch.equal(o1, o2)
+
+
 def test_split_forward_workspace_checked():
     from linatt_amd import _lib
     L, p = _lib.load(), _lib.ptr
