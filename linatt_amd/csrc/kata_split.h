@@ -56,19 +56,22 @@ constexpr int kFwdPart = 32 * 64 + 64;
 constexpr int kMaxPieces = 16;
 
 // A workgroup's time per tile alone on its CU and with the CU full (slots / 256
-// workgroups sharing it), and what a split adds to the call.
+// workgroups sharing it), and what a split adds to the call: once, per piece of
+// the longest list (the second launch adds a block's pieces one after another),
+// and the part of a run that is left uneven at the end.  A split has to be
+// modelled below `win` of the unsplit launch.
 struct TileTime {
   double solo_us, full_us;
   int slots;
-  double split_us;
+  double split_us, piece_us, tail, win;
 };
 
 // Tiles per workgroup with the least modelled time, 0 to leave the launch
 // unsplit.  Modelled as the longer of the longest list at the solo rate and
 // the whole work over all slots at the full rate; for a split the rate of its
-// runs is 1.3 solo and half a run is left uneven at the end, and it adds
-// split_us (the second launch, and the first tile's latency in every workgroup)
-// and the partial blocks written and read at 4.5 TB/s.  It has to win by a tenth.
+// runs is 1.3 solo and `tail` of a run is left uneven at the end, and it adds
+// split_us (the second launch, and the first tile's latency in every workgroup),
+// piece_us per piece and the partial blocks written and read at 4.5 TB/s.
 template <typename Lists>
 inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileTime& tt, double list_bytes) {
   int64_t units = 0;
@@ -80,7 +83,7 @@ inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileT
   }
   const double all = (double)(units * heads) * tt.full_us / tt.slots;
   auto longer = [](double a, double b) { return a > b ? a : b; };
-  double best = 0.9 * longer(longest * tt.solo_us, all);
+  double best = tt.win * longer(longest * tt.solo_us, all);
   int L_best = 0;
   for (int L = 1; L < longest; L = L < 4 ? L + 1 : L + L / 4) {
     if (split_pieces(longest, L) > kMaxPieces) continue;
@@ -89,8 +92,8 @@ inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileT
       const int p = split_pieces(lists(i), L);
       if (p > 1) part += p;
     }
-    const double t = longer(1.3 * L * tt.solo_us, all + 0.5 * L * tt.solo_us) + tt.split_us +
-                     (double)(part * heads) * list_bytes * (2. / 4.5e6);
+    const double t = longer(1.3 * L * tt.solo_us, all + tt.tail * L * tt.solo_us) + tt.split_us +
+                     split_pieces(longest, L) * tt.piece_us + (double)(part * heads) * list_bytes * (2. / 4.5e6);
     if (t < best) {
       best = t;
       L_best = L;
@@ -103,16 +106,21 @@ inline int best_split(const Lists& lists, int64_t heads, int nlists, const TileT
 // three workgroups per CU at dk = 64, two at dk = 128; fp16 adds the row
 // rescaling.  float32: 32 x 32 x 2 products, two workgroups per CU.
 // Unsplit -> split, us: float32 B1 H4 T512 48 -> 17; fp16 M = 2 B1 H12 T3001
-// 57 -> 37; bf16 (with a second launch 3 us slower than now) B1 H12 T2048: sum
-// M = 4 76 -> 40, decayed dk = 128 55 -> 33, concat M = 4 28 -> 26.  Left unsplit: concat M = 4 at B2 T2048 (30 against 33),
-// B4 (39 against 51), M = 1 at B1 T1500 (18 against 19).
+// 57 -> 38; bf16 B1 H12 T2048: sum M = 4 75 -> 39, decayed dk = 128 55 -> 31.
+// The second launch costs 0.2 to 0.4 us per piece; without that term the rule took
+// runs of one or two tiles that were slower than no split (bf16 M = 1 B1 H1 T1000:
+// unsplit 13.3, 16 pieces 15.5, six 10.2; dk = 128 H8 T1000: 17.5, eight pieces
+// 19.3, six 15.0).  Left unsplit: concat M = 4 at B2 T2048 (30 against 33 at the
+// best run length), B4 (39 against 48); and, where the model is on the safe
+// side, B1 H12 T2048 (28 against 23), M = 1 T1500 (18 against 17).
 inline TileTime kata_fwd_tile_time(int elt_bytes, bool fp16, int dk, int M, bool sum, bool decay) {
-  if (elt_bytes == 4) return {6., 14., 512, 8.};
+  if (elt_bytes == 4) return {6., 14., 512, 8., 0., 0.5, 0.9};
   double solo = sum && M > 1 ? (M == 2 ? 1.3 : 2.4) : 0.85;
-  if (dk == 128) solo *= 1.4;
+  if (dk == 128) solo *= decay ? 1.4 : 1.35;
   if (decay) solo *= 1.4;
   if (fp16) solo *= 1.4;
-  return dk == 128 ? TileTime{solo, 1.4 * solo, 512, 8.} : TileTime{solo, 2.2 * solo, 768, 8.};
+  const bool wide = dk == 128;
+  return {solo, (wide ? 1.4 : 2.2) * solo, wide ? 512 : 768, 6.6, 0.2, 0.55, 0.92};
 }
 inline int kata_fwd_split(int64_t BH, int T, const TileTime& tt) {
   return best_split([&](int qt) { return kata_key_tiles(qt, T); }, BH, (T + 127) / 128, tt, 4. * kFwdPart * 4);
@@ -154,16 +162,18 @@ constexpr int kDkdvPart = 32 * 128;
 __host__ __device__ inline int64_t dkdv_part_offset(int piece, int nbk, int bh, int nkt, int blk) {
   return (((int64_t)piece * nbk + bh) * (4 * nkt) + blk) * kDkdvPart;
 }
-// Per 64-query tile of 128 keys, two workgroups per CU.  Unsplit -> split, us
-// (with a second launch 5 to 10 us slower than now):
-// sum M = 2 B6 T1403 HQ12 H4 124 -> 105; concat M = 4 B1 H12 T2048 59 -> 47, B2
-// HQ16 H8 T2048 112 -> 86; M = 1 B1 HQ8 H4 T3000 108 -> 55; sum M = 4 B1 H12
-// T2048 141 -> 90; with the output norm, whole backward, B1 H12 T2048 concat M = 4
-// 111 -> 98, sum M = 4 268 -> 217 (now 93 and 209).  Left unsplit: M = 1 B1 H8
-// T1500 (33 against 35), concat M = 4 B1 H4 T1000 (33 against 34).
+// Per 64-query tile of 128 keys, two workgroups per CU.  Whole backward (dq and
+// dk/dv), unsplit -> split, us: sum M = 2 B6 T1403 HQ12 H4 175 -> 153; concat
+// M = 4 B1 H12 T2048 103 -> 86, B2 HQ16 H8 T2048 161 -> 130, B1 H4 T1000 58 -> 42;
+// M = 1 B1 HQ8 H4 T3000 152 -> 87; sum M = 4 B1 H12 T2048 261 -> 202; with the
+// output norm B1 H12 T2048 concat M = 4 111 -> 93, sum M = 4 269 -> 210.  Left
+// unsplit: concat M = 4 B4 T1024 (63 against 67 at the best run length), B8 T2048
+// (240 against 262); and, where split_us is on the safe side (it was fitted to a
+// second launch 5 to 10 us slower than this one), M = 1 B1 H8 T1500 (58 against 50),
+// concat M = 4 B1 H8 T700 (44 against 36).
 inline TileTime kata_dkdv_tile_time(int M, bool sum) {
   const double full = sum && M > 1 ? (M == 2 ? 3.2 : 7.0) : M == 1 ? 2.1 : M == 2 ? 2.3 : 2.8;
-  return {full / 1.6, full, 512, 13.};
+  return {full / 1.6, full, 512, 13., 0., 0.5, 0.9};
 }
 inline int kata_dkdv_split(int64_t BH, int T, int G, const TileTime& tt) {
   return best_split([&](int st) { return kata_query_tiles(st, T, G); }, BH, (T + 127) / 128, tt, 4. * kDkdvPart * 4);

@@ -192,6 +192,20 @@ def test_bwd_split_workspace_size_checked(lib, B, T, HQ, H, dk, M, variant, dtyp
         assert b"workspace smaller" in lib.linatt_last_error()
 
 
+@pytest.mark.parametrize("H,T,dk,M,most", [(1, 1000, 64, 1, 8), (1, 1000, 64, 2, 8), (4, 1280, 64, 2, 7), (4, 768, 128, 2, 6),
+                                           (8, 1000, 128, 2, 6)])
+def test_forward_split_has_few_pieces_on_short_lists(lib, H, T, dk, M, most):
+    """At these bf16 shapes a split into more than `most` pieces per list was
+    measured slower than the unsplit forward (12 to 16 pieces against 13 to 17
+    us) and one into at most `most` faster: the second launch adds a block's
+    pieces one after another."""
+    nqt = (T + 127) // 128
+    block = (32 * 64 + 64) * 4  # a piece's partial sums of 32 queries, bytes
+    n = lib.linatt_kata_fwd_workspace_bytes(1, T, H, H, dk, 64, M, 0, 0, 1)
+    assert n % (H * 4 * nqt * block) == 0
+    assert n // (H * 4 * nqt * block) <= most
+
+
 def test_python_layer_rejects_cpu_tensors(lib):
     import torch
     from linatt_amd import parallel_kata_attn as P
