@@ -1342,7 +1342,7 @@ static size_t gen_readout_ws(const KataGenStateArgs& a, int ns) {
   return ns > 1 ? (size_t)ns * a.B * a.T * a.H * kGenDecPart * sizeof(float) : 0;
 }
 static size_t gen_update_ws(const KataGenStateArgs& a, int ns) {
-  return ns > 1 ? (size_t)ns * a.B * a.H * a.P * 65 * sizeof(float) : 0;
+  return ns > 1 ? (size_t)ns * a.B * a.H * gen_packed_rows(a) * 65 * sizeof(float) : 0;
 }
 
 static int gen_readout_impl(const char* fn, const void* q, const float* c, const float* S, const float* z,

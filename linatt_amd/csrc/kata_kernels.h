@@ -179,9 +179,11 @@ inline int kata_gen_best_split(int64_t wgs, int steps, double step_us, double pa
 inline bool kata_gen_update_small(int64_t BH, int P) {
   return !(P > 256 || BH * ((P + 255) / 256) >= 512);
 }
-// from the score's packed row count, whatever the state's layout, so that the
-// packed rows equal the full layout's bit for bit (the same sums in the same
-// order)
+// from the score's packed row count, whose partial sums a split writes whatever
+// the state's layout, so that the packed rows equal the full layout's bit for bit
+// (the same sums in the same order).  Partials of all the rows of a full state
+// (about twice as many) made a split of it slower than none at 13 of 540 measured
+// shapes, by up to 22 %.
 inline int kata_gen_update_splits(int64_t BH, int groups, int E, int T) {
   const int P = groups * (E * (E + 1) / 2);
   const int64_t wgs = BH * (kata_gen_update_small(BH, P) ? 2 * ((P + 127) / 128) : (P + 255) / 256);
@@ -226,12 +228,13 @@ struct KataGenStateArgs {
   int TE;            // packed rows per group, E (E + 1) / 2
   int nsplit;        // decode: workgroups per (b, h); update: token splits; readout: row splits (1: direct)
   // nsplit > 1, float32 partials.  decode: (B*H, nsplit, kGenDecPart), num (64)
-  // and den; readout: (nsplit, B, T, H, kGenDecPart) likewise; update:
-  // (nsplit, B*H, P, 64) of S, then (nsplit, B*H, P) of z
+  // and den; readout: (nsplit, B, T, H, kGenDecPart) likewise; update, Pp the
+  // packed rows: (nsplit, B*H, Pp, 64) of S, then (nsplit, B*H, Pp) of z
   float* part;
   float scale, eps;
   int init;          // update: 1 = add to f_T S, 0 = start from zero
 };
+__host__ __device__ inline int gen_packed_rows(const KataGenStateArgs& a) { return (a.sum ? 1 : a.M) * a.TE; }
 enum { KATA_GEN_DECODE = 0, KATA_GEN_READOUT = 1, KATA_GEN_UPDATE = 2 };
 
 template <typename T>

@@ -610,21 +610,32 @@ __global__ __launch_bounds__(256) void kata_gen_update_mfma_kernel(KataGenStateA
 // The split update's state: per state row (16 threads, four columns each) the
 // splits' partial sums added in split order,
 //   S <- (init ? f_T S : 0) + sum_i part_i,  z likewise.
+// The partials are those of the packed rows: a full state's rows (a, b) and
+// (b, a) take the same one (their increments are equal bit for bit), so a split
+// costs it the packed state's products and partial bytes.
 __global__ __launch_bounds__(256) void kata_gen_update_finish_kernel(KataGenStateArgs a) {
   const size_t BH = (size_t)a.B * a.H, rows = BH * a.P;
   const size_t row = (size_t)blockIdx.x * 16 + (threadIdx.x >> 4);
   const int c4 = threadIdx.x & 15;
   if (row >= rows) return;
   const int bh = (int)(row / a.P), b = bh / a.H, h = bh % a.H;
+  const int Pp = gen_packed_rows(a), p = (int)(row % a.P);
+  int pp = p;
+  if (!a.tri) {
+    const RowPair r = row_pair(a, p);
+    const int lo = min(r.a, r.b), hi = max(r.a, r.b);
+    pp = r.g * a.TE + lo * a.E - lo * (lo - 1) / 2 + hi - lo;
+  }
+  const size_t prow = (size_t)bh * Pp + pp, prows = BH * Pp;
   const float fT = a.init ? (a.c ? __expf(a.c[((int64_t)b * a.T + a.T - 1) * a.H + h]) : 1.f) : 0.f;
-  const float* pz = a.part + (size_t)a.nsplit * rows * kGenDV;
+  const float* pz = a.part + (size_t)a.nsplit * prows * kGenDV;
   float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
   float zz = 0.f;
 #pragma unroll 4
   for (int i = 0; i < a.nsplit; ++i) {
-    const float4 y = *reinterpret_cast<const float4*>(a.part + (i * rows + row) * kGenDV + 4 * c4);
+    const float4 y = *reinterpret_cast<const float4*>(a.part + (i * prows + prow) * kGenDV + 4 * c4);
     x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w;
-    if (c4 == 0) zz += pz[i * rows + row];
+    if (c4 == 0) zz += pz[i * prows + prow];
   }
   float4* sp = reinterpret_cast<float4*>(a.S + row * kGenDV + 4 * c4);
   if (a.init) {
@@ -944,12 +955,17 @@ hipError_t launch_kata_gen_state(const KataGenStateArgs& a, int which, hipStream
       kata_gen_readout_kernel<T><<<dim3(BH, (a.T + 63) / 64), dim3(256), 0, stream>>>(a);
     }
   } else if constexpr (sizeof(T) == 2) {
+    KataGenStateArgs u = a;
+    if (a.nsplit > 1) {  // partial sums of the packed rows, whatever the state's layout
+      u.tri = 1;
+      u.P = gen_packed_rows(a);
+    }
     by_sum_groups(a, [&](auto ms) {
       constexpr int MS = decltype(ms)::value;
-      if (kata_gen_update_small(BH, a.P))
-        kata_gen_update_mfma_kernel<T, MS, 1, 1><<<dim3(BH, (a.P + 127) / 128, 2 * a.nsplit), dim3(256), 0, stream>>>(a);
+      if (kata_gen_update_small(BH, u.P))
+        kata_gen_update_mfma_kernel<T, MS, 1, 1><<<dim3(BH, (u.P + 127) / 128, 2 * u.nsplit), dim3(256), 0, stream>>>(u);
       else
-        kata_gen_update_mfma_kernel<T, MS, 2, 2><<<dim3(BH, (a.P + 255) / 256, a.nsplit), dim3(256), 0, stream>>>(a);
+        kata_gen_update_mfma_kernel<T, MS, 2, 2><<<dim3(BH, (u.P + 255) / 256, u.nsplit), dim3(256), 0, stream>>>(u);
       return hipSuccess;
     });
     if (a.nsplit > 1)

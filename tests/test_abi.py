@@ -206,6 +206,18 @@ def test_forward_split_has_few_pieces_on_short_lists(lib, H, T, dk, M, most):
     assert n // (H * 4 * nqt * block) <= most
 
 
+@pytest.mark.parametrize("B,H,T,dk,M,sum_", [(1, 12, 1500, 64, 1, 0), (2, 12, 512, 32, 1, 0), (1, 8, 1000, 64, 2, 1), (1, 12, 1500, 128, 2, 0),
+                                             (1, 2, 300, 16, 1, 0), (16, 8, 1500, 64, 4, 0)])
+def test_split_update_partials_are_the_packed_rows(lib, B, H, T, dk, M, sum_):
+    """A split update writes one partial row per packed row whatever the
+    state's layout: a full state's two rows of a pair share it."""
+    from linatt_amd._lib import LINATT_KATA_PACKED_STATE
+    ws = [lib.linatt_kata_gen_update_workspace_bytes(B, T, H, dk, M, sum_ | v, 1) for v in (0, LINATT_KATA_PACKED_STATE)]
+    assert ws[0] == ws[1] > 0
+    E = dk // M
+    assert ws[0] % (B * H * (1 if sum_ else M) * (E * (E + 1) // 2) * 65 * 4) == 0
+
+
 def test_python_layer_rejects_cpu_tensors(lib):
     import torch
     from linatt_amd import parallel_kata_attn as P
