@@ -1336,7 +1336,7 @@ static int gen_readout_splits(const KataGenStateArgs& a, int dtype) {
   return kata_gen_readout_splits((int64_t)a.B * a.H, a.T, a.E, a.M, a.sum, a.tri);
 }
 static int gen_update_splits(const KataGenStateArgs& a, int dtype) {
-  return half_dtype(dtype) ? kata_gen_update_splits((int64_t)a.B * a.H, a.sum ? 1 : a.M, a.E, a.T) : 1;
+  return half_dtype(dtype) ? kata_gen_update_splits((int64_t)a.B * a.H, a.M, a.sum, a.E, a.T) : 1;
 }
 static size_t gen_readout_ws(const KataGenStateArgs& a, int ns) {
   return ns > 1 ? (size_t)ns * a.B * a.T * a.H * kGenDecPart * sizeof(float) : 0;

@@ -150,17 +150,16 @@ inline int kata_gen_decode_splits(int BH, int P) {
 // dozen such chains.  A split shortens the chain but writes one more partial
 // sum, read back by a second launch: the count taken is the one with the
 // least of chain + second launch + partial bytes, as measured on one MI355X
-// (a chunk 1.9 us; a stage 1.5 us, 0.5 us more per further group of the sum
-// score; the second launch 4 us; the partials at 4.5 TB/s both ways), at most
-// 768 workgroups in all (three per CU, 44-47 KB of LDS each).  B1 H12, us,
+// (the second launch 4 us; the partials at 4.5 TB/s both ways), with at most
+// `slots` workgroups in all, those resident at once.  B1 H12, us,
 // unsplit -> split: update at T = 1500 concat M = 1 47 -> 32, sum M = 4
 // 47 -> 16; readout at T = 200 concat M = 1 62 -> 19; left unsplit, since
 // split it is slower: update at T = 200 concat M = 1 (12 against 17).
 constexpr int kGenMaxSplit = 16;
-inline int kata_gen_best_split(int64_t wgs, int steps, double step_us, double part_bytes) {
+inline int kata_gen_best_split(int64_t wgs, int steps, double step_us, double part_bytes, int slots) {
   int best = 1;
   double t_best = steps * step_us;
-  for (int ns = 2; ns <= kGenMaxSplit && ns <= steps && wgs * ns <= 768; ++ns) {
+  for (int ns = 2; ns <= kGenMaxSplit && ns <= steps && wgs * ns <= slots; ++ns) {
     const int per = (steps + ns - 1) / ns;
     if ((steps + per - 1) / per != ns) continue;  // a split would be empty
     const double t = per * step_us + 4. + ns * part_bytes * (2. / 4.5e6);
@@ -184,15 +183,24 @@ inline bool kata_gen_update_small(int64_t BH, int P) {
 // (the same sums in the same order).  Partials of all the rows of a full state
 // (about twice as many) made a split of it slower than none at 13 of 540 measured
 // shapes, by up to 22 %.
-inline int kata_gen_update_splits(int64_t BH, int groups, int E, int T) {
-  const int P = groups * (E * (E + 1) / 2);
-  const int64_t wgs = BH * (kata_gen_update_small(BH, P) ? 2 * ((P + 127) / 128) : (P + 255) / 256);
-  return kata_gen_best_split(wgs, (T + 63) / 64, 1.9, BH * (P * 260.));
+// A chunk takes 1.9 us, in the small tile 1.6 and 0.1 more per further group of
+// the sum score.  Three workgroups per CU are resident (39-44 KB of LDS, up to 168
+// registers), of the large tile with a sum over 4 or 8 groups two (190
+// registers).  Counting on three, sum M = 4 at dk = 128 was split in two at B16
+// H8 T1500 (92 us, split 107: 768 workgroups of which 512 fit); 1.9 us for every
+// tile split E = 16 at B2 H12 T200 (8.9 us, split 9.3).
+inline int kata_gen_update_splits(int64_t BH, int M, int sum, int E, int T) {
+  const int groups = sum ? M : 1, P = (sum ? 1 : M) * (E * (E + 1) / 2);
+  const bool small = kata_gen_update_small(BH, P);
+  const int64_t wgs = BH * (small ? 2 * ((P + 127) / 128) : (P + 255) / 256);
+  const int slots = !small && (groups == 4 || groups == 8) ? 512 : 768;
+  return kata_gen_best_split(wgs, (T + 63) / 64, small ? 1.6 + 0.1 * (groups - 1) : 1.9, BH * (P * 260.), slots);
 }
 inline int kata_gen_readout_splits(int64_t BH, int T, int E, int M, int sum, int tri) {
-  // stages of four 16-row chunks (readout_chunk)
+  // stages of four 16-row chunks (readout_chunk): 1.5 us each, 0.5 us more per
+  // further group of the sum score; three workgroups per CU (47-53 KB of LDS)
   const int stages = (sum ? 1 : M) * (tri ? E * (E + 16) / 32 : E * (E / 16)) / 4;
-  return kata_gen_best_split(BH * ((T + 127) / 128), stages, 1.5 + (sum ? 0.5 * (M - 1) : 0.), BH * (T * 272.));
+  return kata_gen_best_split(BH * ((T + 127) / 128), stages, 1.5 + (sum ? 0.5 * (M - 1) : 0.), BH * (T * 272.), 768);
 }
 
 struct KataDecodeArgs {

@@ -218,6 +218,15 @@ def test_split_update_partials_are_the_packed_rows(lib, B, H, T, dk, M, sum_):
     assert ws[0] % (B * H * (1 if sum_ else M) * (E * (E + 1) // 2) * 65 * 4) == 0
 
 
+@pytest.mark.parametrize("B,H,T,dk,M,sum_", [(8, 12, 1500, 128, 4, 1), (8, 12, 2000, 128, 4, 1), (16, 8, 1500, 128, 4, 1), (16, 8, 2000, 128, 4, 1),
+                                             (2, 12, 200, 16, 1, 0)])
+def test_update_not_split_where_split_is_slower(lib, B, H, T, dk, M, sum_):
+    """bf16 prompts into an empty cache whose split update was measured slower
+    (the first: 92 us unsplit, 98 split; the last 8.9 and 9.3)."""
+    from linatt_amd._lib import LINATT_KATA_PACKED_STATE
+    assert lib.linatt_kata_gen_update_workspace_bytes(B, T, H, dk, M, sum_ | LINATT_KATA_PACKED_STATE, 1) == 0
+
+
 def test_python_layer_rejects_cpu_tensors(lib):
     import torch
     from linatt_amd import parallel_kata_attn as P
