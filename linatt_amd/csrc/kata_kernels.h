@@ -150,19 +150,21 @@ inline int kata_gen_decode_splits(int BH, int P) {
 // dozen such chains.  A split shortens the chain but writes one more partial
 // sum, read back by a second launch: the count taken is the one with the
 // least of chain + second launch + partial bytes, as measured on one MI355X
-// (the second launch 4 us; the partials at 4.5 TB/s both ways), with at most
-// `slots` workgroups in all, those resident at once.  B1 H12, us,
+// (finish_us the second launch; the partials at 4.5 TB/s both ways), below `win` of
+// the unsplit chain, with at most `slots` workgroups in all, those resident at
+// once.  B1 H12, us,
 // unsplit -> split: update at T = 1500 concat M = 1 47 -> 32, sum M = 4
 // 47 -> 16; readout at T = 200 concat M = 1 62 -> 19; left unsplit, since
 // split it is slower: update at T = 200 concat M = 1 (12 against 17).
 constexpr int kGenMaxSplit = 16;
-inline int kata_gen_best_split(int64_t wgs, int steps, double step_us, double part_bytes, int slots) {
+inline int kata_gen_best_split(int64_t wgs, int steps, double step_us, double part_bytes, int slots,
+                               double finish_us, double win) {
   int best = 1;
-  double t_best = steps * step_us;
+  double t_best = win * steps * step_us;
   for (int ns = 2; ns <= kGenMaxSplit && ns <= steps && wgs * ns <= slots; ++ns) {
     const int per = (steps + ns - 1) / ns;
     if ((steps + per - 1) / per != ns) continue;  // a split would be empty
-    const double t = per * step_us + 4. + ns * part_bytes * (2. / 4.5e6);
+    const double t = per * step_us + finish_us + ns * part_bytes * (2. / 4.5e6);
     if (t < t_best) {
       t_best = t;
       best = ns;
@@ -194,13 +196,18 @@ inline int kata_gen_update_splits(int64_t BH, int M, int sum, int E, int T) {
   const bool small = kata_gen_update_small(BH, P);
   const int64_t wgs = BH * (small ? 2 * ((P + 127) / 128) : (P + 255) / 256);
   const int slots = !small && (groups == 4 || groups == 8) ? 512 : 768;
-  return kata_gen_best_split(wgs, (T + 63) / 64, small ? 1.6 + 0.1 * (groups - 1) : 1.9, BH * (P * 260.), slots);
+  return kata_gen_best_split(wgs, (T + 63) / 64, small ? 1.6 + 0.1 * (groups - 1) : 1.9, BH * (P * 260.), slots, 4.,
+                             1.);
 }
 inline int kata_gen_readout_splits(int64_t BH, int T, int E, int M, int sum, int tri) {
   // stages of four 16-row chunks (readout_chunk): 1.5 us each, 0.5 us more per
-  // further group of the sum score; three workgroups per CU (47-53 KB of LDS)
+  // further group of the sum score up to five; three workgroups per CU (47-53 KB of
+  // LDS).  Long chunks' partials (272 bytes per query and split) pay only for a
+  // clear win: taken at a modelled tie, B1 H8 T4096 sum M = 2 went from 26.5 to
+  // 31.1 us, sum M = 8 at dk = 128 (2 us for a group more each) from 18.5 to 22
   const int stages = (sum ? 1 : M) * (tri ? E * (E + 16) / 32 : E * (E / 16)) / 4;
-  return kata_gen_best_split(BH * ((T + 127) / 128), stages, 1.5 + (sum ? 0.5 * (M - 1) : 0.), BH * (T * 272.), 768);
+  const double step = 1.5 + (sum ? 0.5 * (M < 5 ? M - 1 : 4) : 0.);
+  return kata_gen_best_split(BH * ((T + 127) / 128), stages, step, BH * (T * 272.), 768, 3.5, 0.97);
 }
 
 struct KataDecodeArgs {

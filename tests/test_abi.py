@@ -227,6 +227,14 @@ def test_update_not_split_where_split_is_slower(lib, B, H, T, dk, M, sum_):
     assert lib.linatt_kata_gen_update_workspace_bytes(B, T, H, dk, M, sum_ | LINATT_KATA_PACKED_STATE, 1) == 0
 
 
+@pytest.mark.parametrize("B,H,T,dk,M,sum_", [(1, 8, 4096, 64, 4, 0), (1, 8, 4096, 64, 2, 1), (1, 4, 4096, 128, 8, 1), (4, 12, 400, 128, 8, 1)])
+def test_readout_not_split_where_split_is_slower(lib, B, H, T, dk, M, sum_):
+    """bf16 chunks whose split readout was measured 8 to 24 % slower (29 us
+    unsplit, 32 split; 26.5 and 31; 18.4 and 21.8; 19.2 and 23.5)."""
+    from linatt_amd._lib import LINATT_KATA_PACKED_STATE
+    assert lib.linatt_kata_gen_readout_workspace_bytes(B, T, H, dk, M, sum_ | LINATT_KATA_PACKED_STATE, 1) == 0
+
+
 def test_python_layer_rejects_cpu_tensors(lib):
     import torch
     from linatt_amd import parallel_kata_attn as P
