@@ -342,10 +342,14 @@ def test_split_decode_equals_decode(dk, M, variant, packed, decay):
 @pytest.mark.parametrize("T", [1, 64, 255, 257, 1500])
 def test_split_update_readout_equal_unsplit(dk, M, variant, packed, decay, dtype, T):
     """``linatt_kata_gen_update_split`` / ``_readout_split`` against the
-    unsplit calls, from a stored state: the same products, summed in another
-    order.  Bounds: two float32 sums of n terms differ by at most
-    2 n 2^-24 sum|terms| (S, z, and with them den); o is rounded once more to
-    the dtype (one spacing, 2^-7 bf16 / 2^-10 fp16 of the value)."""
+    unsplit calls, from a stored state: the same products (of 16-bit rounded
+    factors, at most 1 + 2^-6 of the exact ones), summed in another order.
+    Bounds, value by value: two float32 sums of n terms differ by at most
+    2 n 2^-24 sum|terms|, the sums of absolute terms taken in float64 from the
+    features themselves (S, z and den; o = num / den with both sums' errors);
+    o is rounded once more to the dtype (one spacing, 2^-7 bf16 / 2^-10 fp16
+    of the value).  The readout's bounds are shown to tell: without any one
+    sixteenth of the state's rows, num and den move by more."""
     from linatt_amd import _lib
     from linatt_amd.kata_cache import state_rows
     B, H, E = 1, 3, dk // M
@@ -365,8 +369,10 @@ def test_split_update_readout_equal_unsplit(dk, M, variant, packed, decay, dtype
                                              dk, 64, M, var, sc, code, sp))
     ru = L.linatt_kata_gen_update_workspace_bytes(B, T, H, dk, M, var, code)
     rr = L.linatt_kata_gen_readout_workspace_bytes(B, T, H, dk, M, var, code)
-    # a long call of every score splits; how short a call still does depends on the partials' size
+    # a long call of every score splits its update; how short a call still does depends on the partials'
+    # size.  The readout splits but where four stages of rows (E = 16, one group) meet a long call's partials
     assert ru > 0 or T <= 257
+    assert rr > 0 or (dk == 16 and T == 1500)
     out = []
     for split in (False, True):
         S, z, o, den = S0.clone(), z0.clone(), o0.clone(), den0.clone()
@@ -384,18 +390,37 @@ def test_split_update_readout_equal_unsplit(dk, M, variant, packed, decay, dtype
                                                      code, sp))
         out.append((S, z, o, den))
     torch.cuda.synchronize()
-    (S1, z1, o1, d1), (S2, z2, o2, d2) = out
-    # sum|terms| over the largest feature of any row: |psi| <= M scale max|k|^2
-    fmax = M * sc * k.float().abs().amax() ** 2
-    n = T + 66
-    tol = 2 * n * 2.0 ** -24 * (T * fmax * v.float().abs().amax() + S0.abs().amax())
-    assert (S1 - S2).abs().max() <= tol
-    assert (z1 - z2).abs().max() <= 2 * n * 2.0 ** -24 * (T * fmax + z0.abs().amax())
-    qf = M * sc * q.float().abs().amax() ** 2
-    nr = P + 66
-    den_tol = 2 * nr * 2.0 ** -24 * (2 * P * qf * z0.abs().amax() + den0.abs().amax())
-    assert (d1 - d2).abs().max() <= den_tol
+    (S1, z1, o1, d1), (S2, z2, o2, d2) = (tuple(x[0].double() for x in y) for y in out)
+    a, b = torch.triu_indices(E, E, device="cuda") if packed else torch.cartesian_prod(*[torch.arange(E, device="cuda")] * 2).t()
+
+    def psi(x, weight):  # (T, H, dk) -> (H, T, P)
+        xg = x[0].double().transpose(0, 1).reshape(H, T, M, E)
+        f = sc * xg[..., a] * xg[..., b]
+        f = f.sum(2) if variant == "sum" else f.flatten(2)
+        return f * torch.where(a == b, 1.0, 2.0).double().repeat(1 if variant == "sum" else M) if weight and packed else f
+
+    slack = 1 + 2.0 ** -6
+    eps = 2 * (T + 66) * 2.0 ** -24 * slack
+    f = psi(k, False).abs()
+    fT = torch.ones(H, device="cuda").double()
+    if decay:
+        f = f * torch.exp(c[0, -1].double() - c[0].double()).t()[..., None]
+        fT = torch.exp(c[0, -1].double())
+    Sz, zz = S0[0].double(), z0[0].double()
+    fv = f.transpose(1, 2).contiguous()
+    assert ((S1 - S2).abs() <= eps * (fv @ v[0].double().abs().transpose(0, 1).contiguous() + fT[:, None, None] * Sz.abs())).all()
+    assert ((z1 - z2).abs() <= eps * (f.sum(1) + fT[:, None] * zz.abs())).all()
+    # readout, (H, T, ...)
+    eps = 2 * (P + 66) * 2.0 ** -24 * slack
+    f = psi(q, True)
+    fd = torch.exp(c[0].double()).t() if decay else torch.ones(H, T, device="cuda").double()
+    o1, o2, d1, d2, o0, den0 = (x.transpose(0, 1) for x in (o1, o2, d1, d2, o0[0].double(), den0[0].double()))
+    den_tol = eps * (fd * (f.abs() @ zz[..., None].abs())[..., 0] + den0)
+    assert ((d1 - d2).abs() <= den_tol).all()
+    num_tol = eps * (fd[..., None] * (f.abs() @ Sz.abs()) + (o0.abs() * den0[..., None]))
     spacing = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
-    num_tol = 2 * nr * 2.0 ** -24 * (2 * P * qf * S0.abs().amax() + (o0.float().abs() * den0[..., None]).amax())
-    o_tol = spacing * o1.float().abs() + ((num_tol + o1.float().abs() * den_tol) / d1[..., None])
-    assert ((o1.float() - o2.float()).abs() <= o_tol).all()
+    assert ((o1 - o2).abs() <= spacing * o1.abs() + (num_tol + o1.abs() * den_tol[..., None]) / d1[..., None]).all()
+    for run in torch.arange(P, device="cuda").chunk(16):
+        num = fd[..., None] * (f[..., run] @ Sz[:, run])
+        assert (num.abs() > num_tol + spacing * o1.abs() * d1[..., None]).any()
+        assert ((fd * (f[..., run] * zz[:, None, run]).sum(-1)).abs() > den_tol).any()
