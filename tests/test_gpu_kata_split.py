@@ -93,6 +93,95 @@ def test_split_forward_fp16_tiny_weights():
     assert torch.equal(d1, d2) and torch.equal(o1, o2)
 
 
+def _special(q, k, v):
+    """Rows without weights (zero queries, the first key included), then a NaN
+    key and an infinite value, each well inside a cut list."""
+    T = q.shape[1]
+    q[:, 0] = q[:, 700:760] = 0
+    k[:, T // 2 + 7, 0, 3] = float("nan")
+    v[:, T // 2 - 130, -1, 5] = float("inf")
+
+
+def _same_special(a, b, tol):
+    a, b = a.double(), b.double()
+    assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
+    fin = a.isfinite()
+    assert fin.any() and not fin.all()
+    assert torch.equal(a[a.isinf()], b[a.isinf()])
+    a, b = torch.where(fin, a, 0.0), torch.where(fin, b, 0.0)
+    assert ((a - b).abs() <= tol(a)).all()
+
+
+@pytest.mark.parametrize("T,HQ,H,dk,M,variant,decay,dtype", [
+    (2049, 3, 3, 64, 4, "sum", False, torch.bfloat16), (2600, 4, 2, 64, 4, "concat", False, torch.bfloat16),
+    (3100, 2, 2, 64, 2, "concat", True, torch.float16), (2100, 2, 2, 128, 2, "sum", False, torch.float16),
+    (2000, 4, 2, 64, 2, "concat", False, torch.float32)])
+def test_split_forward_special_values(T, HQ, H, dk, M, variant, decay, dtype):
+    """Zero denominators, NaN and infinities come out of the split forward where
+    the unsplit one has them, and nowhere else."""
+    from linatt_amd import _lib
+    print(f"\nsplit forward, special values, T{T} HQ{HQ} H{H} dk{dk} M{M} {variant} decay={decay} {dtype}", flush=True)
+    L, p = _lib.load(), _lib.ptr
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(1, T, HQ, dk, generator=g).to(dtype).cuda()
+    k, v = (torch.randn(1, T, H, d, generator=g).to(dtype).cuda() for d in (dk, 64))
+    _special(q, k, v)
+    c = (-torch.rand(1, T, HQ, generator=g) * 0.05).cumsum(1).cuda() if decay else None
+    var, code, shape = int(variant == "sum"), _lib.dtype_code(dtype), (1, T, HQ, H, dk, 64, M)
+    nws = L.linatt_kata_fwd_workspace_bytes(*shape, var, int(decay), code)
+    assert nws > 0
+    ws = torch.empty(nws, device="cuda", dtype=torch.uint8)
+    out = []
+    for split in (False, True):
+        o, den = torch.empty(1, T, HQ, 64, device="cuda", dtype=dtype), torch.empty(1, T, HQ, device="cuda")
+        head, tail = (p(q), p(k), p(v), p(c), p(o), p(den)), (*shape, 1 / math.sqrt(dk // M), var, code, _lib.stream_of(q))
+        if split:
+            _lib.check("split", L.linatt_kata_fwd_split(*head, p(ws), nws, *tail))
+        else:
+            _lib.check("fwd", L.linatt_kata_fwd(*head, *tail))
+        out.append((o, den))
+    torch.cuda.synchronize()
+    (o1, d1), (o2, d2) = out
+    assert (d1[:, 700:760] == 0).all() and (o1[:, 700:760].float() == 0).all()
+    vmax = v[v.isfinite()].double().abs().max()
+    acc = 2 * T * 2.0 ** -24 + (2.0 ** -10 if dtype == torch.float16 else 0.0)
+    _same_special(d1, d2, lambda a: acc * a)
+    _same_special(o1, o2, lambda a: SPACING[dtype] * a.abs() + 2 * acc * vmax)
+
+
+@pytest.mark.parametrize("B,T,HQ,H,M,variant", [(1, 2048, 3, 3, 4, "concat"), (1, 1985, 6, 2, 1, "concat"), (1, 1930, 2, 1, 4, "sum")])
+def test_split_backward_special_values(B, T, HQ, H, M, variant):
+    """The same for dk and dv (bounds as in the plain comparison)."""
+    from linatt_amd import _lib
+    print(f"\nsplit backward, special values, B{B} T{T} HQ{HQ} H{H} M{M} {variant}", flush=True)
+    L, p = _lib.load(), _lib.ptr
+    g = torch.Generator().manual_seed(T + M)
+    q, do = (torch.randn(B, T, HQ, 64, generator=g).bfloat16().cuda() for _ in range(2))
+    k, v = (torch.randn(B, T, H, 64, generator=g).bfloat16().cuda() for _ in range(2))
+    o, den = torch.empty_like(q), torch.empty(B, T, HQ, device="cuda")
+    var, sp, sc, shape = int(variant == "sum"), _lib.stream_of(q), math.sqrt(M) / 8, (B, T, HQ, H, 64, 64, M)
+    q[:, 0] = q[:, 700:760] = 0
+    _lib.check("fwd", L.linatt_kata_fwd(p(q), p(k), p(v), None, p(o), p(den), *shape, sc, var, 1, sp))
+    do[:, T // 2 + 7, 0, 3], do[:, T // 3, -1, 5] = float("nan"), float("inf")
+    ns = L.linatt_kata_bwd_split_workspace_bytes(*shape, var, 1)
+    assert ns > L.linatt_kata_bwd_workspace_bytes(B, T, HQ, 64, 1) + 256  # the split engages
+    ws = torch.empty(ns, device="cuda", dtype=torch.uint8)
+    out = []
+    for split in (False, True):
+        gr = [torch.empty_like(x) for x in (q, k, v)]
+        head, tail = (p(q), p(k), p(v), p(o), p(den), p(do), *map(p, gr), p(ws)), (*shape, sc, var, 1, sp)
+        if split:
+            _lib.check("split", L.linatt_kata_bwd_split(*head, ns, *tail))
+        else:
+            _lib.check("bwd", L.linatt_kata_bwd(*head, *tail))
+        out.append(gr)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0][0].isnan(), out[1][0].isnan())
+    for a, b in zip(out[0][1:], out[1][1:]):
+        top = a[a.isfinite()].double().abs().max()
+        _same_special(a, b, lambda x: 2.0 ** -7 * x.abs() + 2.0 ** -12 * top)
+
+
 def test_split_forward_workspace_checked():
     from linatt_amd import _lib
     L, p = _lib.load(), _lib.ptr
