@@ -233,15 +233,19 @@ def bench_kata_variant(steps, settle_s, B, H, T, dk, dv, M, variant, decay, seed
     den = torch.empty(B, T, H, device=dev)
     dq, dk_, dv_ = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     dc = torch.empty_like(c) if decay else None
-    ws = torch.empty(L.linatt_kata_bwd_workspace_bytes(B, T, H, dv, _lib.LINATT_BFLOAT16),
-                     device=dev, dtype=torch.uint8)
     P, bt, sp = _lib.ptr, _lib.LINATT_BFLOAT16, _lib.stream_of(q)
     scale = 1.0 / math.sqrt(dk // M)
     var = 1 if variant == "sum" else 0
+    # the entries the Python layer calls (they split a launch that leaves CUs idle)
+    shape = (B, T, H, H, dk, dv, M)
+    nf = L.linatt_kata_fwd_workspace_bytes(*shape, var, int(decay), bt)
+    nb = (L.linatt_kata_bwd_workspace_bytes(B, T, H, dv, bt) if decay
+          else L.linatt_kata_bwd_split_workspace_bytes(*shape, var, bt))
+    wf, ws = (torch.empty(n, device=dev, dtype=torch.uint8) for n in (nf, nb))
 
     def fwd():
-        _lib.check("linatt_kata_fwd", L.linatt_kata_fwd(
-            P(q), P(k), P(v), P(c), P(o), P(den), B, T, H, H, dk, dv, M, scale, var, bt, sp))
+        _lib.check("linatt_kata_fwd_split", L.linatt_kata_fwd_split(
+            P(q), P(k), P(v), P(c), P(o), P(den), P(wf), nf, *shape, scale, var, bt, sp))
 
     def bwd():
         if decay:
@@ -249,9 +253,9 @@ def bench_kata_variant(steps, settle_s, B, H, T, dk, dv, M, variant, decay, seed
                 P(q), P(k), P(v), P(c), P(o), P(den), P(do), P(dq), P(dk_), P(dv_), P(dc), P(ws),
                 B, T, H, H, dk, dv, M, scale, bt, sp))
         else:
-            _lib.check("linatt_kata_bwd", L.linatt_kata_bwd(
-                P(q), P(k), P(v), P(o), P(den), P(do), P(dq), P(dk_), P(dv_), P(ws),
-                B, T, H, H, dk, dv, M, scale, var, bt, sp))
+            _lib.check("linatt_kata_bwd_split", L.linatt_kata_bwd_split(
+                P(q), P(k), P(v), P(o), P(den), P(do), P(dq), P(dk_), P(dv_), P(ws), nb,
+                *shape, scale, var, bt, sp))
 
     per, ms = _time_parts([("fwd", fwd), ("bwd", bwd)], steps, settle_s)
     fl = kata_flops(B, H, T, dk, dv, M, variant)
@@ -285,7 +289,12 @@ def bench_kata_onorm(steps, settle_s, M=4):
     dw = torch.empty(D, device=dev)
     bt = _lib.LINATT_BFLOAT16
     n = B * T * H
-    ws = torch.empty(L.linatt_kata_bwd_onorm_workspace_bytes(B, T, H, D, bt), device=dev, dtype=torch.uint8)
+    # the entries the Python layer calls
+    shape = (B, T, H, H, D, D, M)
+    nf = L.linatt_kata_fwd_workspace_bytes(*shape, 0, 0, bt)
+    nb = L.linatt_kata_bwd_split_workspace_bytes(*shape, 0, bt)
+    no = L.linatt_kata_bwd_onorm_split_workspace_bytes(*shape, 0, 0, bt)
+    wf, ws = (torch.empty(x, device=dev, dtype=torch.uint8) for x in (nf, max(nb, no)))
     rws = torch.empty(L.linatt_rmsnorm_bwd_workspace_bytes(n, D), device=dev, dtype=torch.uint8)
     P, sp, scale = _lib.ptr, _lib.stream_of(q), 1.0 / math.sqrt(D // M)
 
@@ -295,22 +304,21 @@ def bench_kata_onorm(steps, settle_s, M=4):
             scale, 0, bt, sp))
 
     def f_bwd():
-        _lib.check("linatt_kata_bwd_onorm", L.linatt_kata_bwd_onorm(
+        _lib.check("linatt_kata_bwd_onorm_split", L.linatt_kata_bwd_onorm_split(
             P(q), P(k), P(v), None, P(o), P(den), P(rstd), P(w), P(dy), P(dq), P(dk), P(dv), None,
-            P(dw), P(ws), B, T, H, H, D, D, M, scale, 0, bt, sp))
+            P(dw), P(ws), no, *shape, scale, 0, bt, sp))
 
     def u_fwd():
-        _lib.check("linatt_kata_fwd", L.linatt_kata_fwd(
-            P(q), P(k), P(v), None, P(o), P(den), B, T, H, H, D, D, M, scale, 0, bt, sp))
+        _lib.check("linatt_kata_fwd_split", L.linatt_kata_fwd_split(
+            P(q), P(k), P(v), None, P(o), P(den), P(wf), nf, *shape, scale, 0, bt, sp))
         _lib.check("linatt_rmsnorm_fwd", L.linatt_rmsnorm_fwd(
             P(o), P(w), P(y), P(rstd), n, D, 1e-5, bt, sp))
 
     def u_bwd():
         _lib.check("linatt_rmsnorm_bwd", L.linatt_rmsnorm_bwd(
             P(o), P(w), P(rstd), P(dy), P(dO), P(dw), P(rws), n, D, bt, sp))
-        _lib.check("linatt_kata_bwd", L.linatt_kata_bwd(
-            P(q), P(k), P(v), P(o), P(den), P(dO), P(dq), P(dk), P(dv), P(ws),
-            B, T, H, H, D, D, M, scale, 0, bt, sp))
+        _lib.check("linatt_kata_bwd_split", L.linatt_kata_bwd_split(
+            P(q), P(k), P(v), P(o), P(den), P(dO), P(dq), P(dk), P(dv), P(ws), nb, *shape, scale, 0, bt, sp))
 
     pf, msf = _time_parts([("fwd", f_fwd), ("bwd", f_bwd)], steps, settle_s)
     pu, msu = _time_parts([("fwd", u_fwd), ("bwd", u_bwd)], steps, settle_s / 2)
@@ -906,7 +914,8 @@ def cpu_baseline_delta(gated, seconds):
 
 def bench_config1(steps):
     """Config 1 on the GPU: the fp32 KATA forward at (1, 512, 4, 64), M=4,
-    q, k, v i.i.d. N(0,1) (seed 0), through linatt_kata_fwd."""
+    q, k, v i.i.d. N(0,1) (seed 0), through linatt_kata_fwd_split (the entry the
+    Python layer calls)."""
     import torch
     from linatt_amd import _lib
     L = _lib.load()
@@ -919,10 +928,13 @@ def bench_config1(steps):
     den = torch.empty(B, T, H, device=dev)
     sp = _lib.stream_of(qd)
     P = _lib.ptr
+    shape = (B, T, H, H, D, D, M)
+    nf = L.linatt_kata_fwd_workspace_bytes(*shape, 0, 0, _lib.LINATT_FLOAT32)
+    wf = torch.empty(nf, device=dev, dtype=torch.uint8)
 
     def fwd():
-        _lib.check("linatt_kata_fwd", L.linatt_kata_fwd(
-            P(qd), P(kd), P(vd), None, P(o), P(den), B, T, H, H, D, D, M, 1.0 / math.sqrt(D // M),
+        _lib.check("linatt_kata_fwd_split", L.linatt_kata_fwd_split(
+            P(qd), P(kd), P(vd), None, P(o), P(den), P(wf), nf, *shape, 1.0 / math.sqrt(D // M),
             0, _lib.LINATT_FLOAT32, sp))
 
     for _ in range(3):
