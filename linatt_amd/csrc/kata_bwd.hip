@@ -1084,11 +1084,13 @@ __global__ __launch_bounds__(64 * kata_dkdv_waves<DK>(), 2) void kata_bwd_dkdv_t
   // units: the next unit's score and the previous one's dK product are issued
   // under this unit's VALU work, block 1's x chain under block 0's last units
   // and block 0's dV products under block 1's first; the fences keep that
-  // order.  VALU-bound with the MFMA issue (204 VALU and 20 MFMA a block at M =
-  // 4, most of which the two waves per SIMD now overlap).  B8 H12 T2048, the
-  // serial body with operands in LDS -> this: M = 4 148 -> 142 us, M = 2
-  // 123 -> 116, M = 1 114 -> 108, sum M = 4 387 -> 358.  A third ring slot
-  // spills (M = 4 170 us).
+  // order.  VALU-bound with the MFMA issue, 12.3 VALU instructions per MFMA at
+  // M = 4; by the counters a SIMD spends 191 k cycles on VALU and 100 k on MFMA
+  // in a launch of 315 k, so the two still overlap little (the serial body: the
+  // same counts in 334 k).  B8 H12 T2048, the serial body with operands in LDS ->
+  // this: M = 4 148 -> 142 us, M = 2 123 -> 116, M = 1 114 -> 108, sum M = 4
+  // 387 -> 358 (which spills two registers, in a split launch four).  A third
+  // ring slot spills (M = 4 170 us).
   auto tile_pipe = [&](int n) __attribute__((always_inline)) {
     constexpr int NU = SUM ? M * M : M;
     const int buf = n % NB;

@@ -295,8 +295,11 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void kata_fwd_kernel(
 // EPI: 0 writes o; 1 also the output RMSNorm's y and rstd; 2 the float32
 // numerator o den instead of o; 3 the workgroup's share of a split launch
 // (kata_split.h: its run of key tiles, and partial rows where the list was
-// cut) (compile-time, so each variant carries only its own epilogue).  Three waves per SIMD at dk = 64 (at most 168 VGPRs;
-// the compiler otherwise lets some variants grow just past it)
+// cut) (compile-time, so each variant carries only its own epilogue).  Three
+// waves per SIMD at dk = 64 (at most 168 VGPRs; the compiler otherwise lets some
+// variants grow just past it).  Under that cap EPI 3 spills 18 registers at
+// concat M = 4 and 10 at M = 2 in bf16, where EPI 0 spills none: the rule's
+// figures for these are of that kernel.
 template <typename T, int DK, int DV, int M, bool SUM, bool DECAY, int EPI>
 __global__ __launch_bounds__(256, DK == 64 ? 3 : 2) void kata_fwd_tile_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
